@@ -17,6 +17,7 @@
 
 #include "../../include/aether_fabric.h"
 #include "engine_internal.hpp"
+#include "prefill_kernels.hpp"
 #include "weaver_kernels.hpp"
 
 static_assert(sizeof(aw_sparse_code) == 16, "SparseCode is 16 bytes (types.rs:227)");
@@ -793,6 +794,26 @@ int launch_finish(aw_engine* e, const aw_decode_desc* d, const Layout& o, char* 
 }
 
 template <int HD>
+int enqueue_merge(aw_engine* e, const aw::MergeArgs& a, hipStream_t st) {
+    const uint64_t gx = cdiv(a.total_rows, 4);
+    if (gx > 0x7FFFFFFFull) return fail(e, AW_E_UNSUPPORTED, "merge grid too large");
+    StageTimer t(e, AW_STAGE_MERGE, st);
+    // Deep load batches when the rows have many partials (measured at B = 1: 45.2 us
+    // a step with 16 float4 loads per batch, 45.9 with 8), shallow ones otherwise
+    // (B = 64: 16 ranges, 2 hot splits).
+    if (a.total_rows <= 4ull * e->n_cu && (a.n_ar > 8 || a.hot_splits > 8))
+        // Few rows with many partials: a work-group per row, its waves splitting them
+        // (measured to B = 32; B = 8 step 58.2 -> 55.8 us).
+        hipLaunchKernelGGL((aw::merge_row_kernel<HD, 8>), dim3((uint32_t)a.total_rows), dim3(256), 0, st, a);
+    else if (a.n_ar > 16 || a.hot_splits > 8)
+        hipLaunchKernelGGL((aw::merge_kernel<HD, 16>), dim3((uint32_t)gx), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((aw::merge_kernel<HD, 4>), dim3((uint32_t)gx), dim3(256), 0, st, a);
+    AW_HIP(e, hipGetLastError());
+    return AW_OK;
+}
+
+template <int HD>
 int launch_merge(aw_engine* e, const aw_decode_desc* d, const Layout& o, char* ws, hipStream_t st) {
     aw::MergeArgs a{};
     const bool cold = o.info.cold_splits > 0 && !o.cold_out; // value partials come in as splits of the hot arrays
@@ -816,22 +837,7 @@ int launch_merge(aw_engine* e, const aw_decode_desc* d, const Layout& o, char* w
     a.hot_splits = o.part_splits;
     a.n_ar = cold ? o.n_ar : 0u;
     a.total_rows = (uint64_t)d->layers * d->batch * d->kv_heads * a.rows_r;
-    const uint64_t gx = cdiv(a.total_rows, 4);
-    if (gx > 0x7FFFFFFFull) return fail(e, AW_E_UNSUPPORTED, "merge grid too large");
-    StageTimer t(e, AW_STAGE_MERGE, st);
-    // Deep load batches when the rows have many partials (measured at B = 1: 45.2 us
-    // a step with 16 float4 loads per batch, 45.9 with 8), shallow ones otherwise
-    // (B = 64: 16 ranges, 2 hot splits).
-    if (a.total_rows <= 4ull * e->n_cu && (a.n_ar > 8 || a.hot_splits > 8))
-        // Few rows with many partials: a work-group per row, its waves splitting them
-        // (measured to B = 32; B = 8 step 58.2 -> 55.8 us).
-        hipLaunchKernelGGL((aw::merge_row_kernel<HD, 8>), dim3((uint32_t)a.total_rows), dim3(256), 0, st, a);
-    else if (a.n_ar > 16 || a.hot_splits > 8)
-        hipLaunchKernelGGL((aw::merge_kernel<HD, 16>), dim3((uint32_t)gx), dim3(256), 0, st, a);
-    else
-        hipLaunchKernelGGL((aw::merge_kernel<HD, 4>), dim3((uint32_t)gx), dim3(256), 0, st, a);
-    AW_HIP(e, hipGetLastError());
-    return AW_OK;
+    return enqueue_merge<HD>(e, a, st);
 }
 
 // Stage order on `st`: [q.D^T] -> cold -> finish [-> merge], or [q.D^T] ->
@@ -915,6 +921,87 @@ int decode_device(aw_engine* e, const aw_decode_desc* d, hipStream_t st, bool no
     if ((rc = ensure_keep(e->ws, o.info.workspace_bytes, e->retired_ws, e->last_error, st))) return rc;
     char* ws = (char*)e->ws.ptr;
     return d->head_dim == 64 ? run_pipeline<64>(e, d, o, ws, st) : run_pipeline<128>(e, d, o, ws, st);
+}
+
+// Key splits of prefill_kernel: each row tile's positions are cut into `splits`
+// parts when that shortens the call by more than the merge of the parts costs.
+// The estimate (us, fitted to this GPU at both head dims, 64 .. 8192 rows per kv
+// head and 64 .. 5000 positions): a 64-position step takes `one` with one
+// work-group per CU and `two` with two, which fill the CU; a merge 4 us and 0.35 ns
+// a row plus 0.16 ns per part of 128 dims.  Measured, 509 queries of 14 heads
+// behind 1022 positions (56 work-groups of 24 steps): 1 part 24.3 us, 2 21.8, 4
+// 19.5, 8 22.1; 17 queries of 32 heads over 4096 positions: 1 part 82, 4 28, 16
+// 15.6, 32 15.7; 512 of 32 over 512: 1 part 16.3, 2 28.9.
+uint32_t prefill_splits(uint64_t items, uint32_t steps, uint64_t rows, int HD, uint32_t n_cu) {
+    const double one = HD == 128 ? 1.5 : 1.0, two = HD == 128 ? 2.6 : 1.8;
+    uint32_t best = 1;
+    double best_us = 0.0;
+    for (uint32_t s = 1; s <= std::min<uint32_t>(steps, aw::kMaxSplits); s *= 2) {
+        const uint64_t wgs = items * s;
+        if (s > 1 && wgs > 4ull * n_cu) break; // parts of at most 64 MiB (128 dims, 256 CUs)
+        const double rounds = std::max(1.0, (double)wgs / (2.0 * n_cu));
+        double us = cdiv(steps, s) * (wgs <= n_cu ? one : two * rounds);
+        if (s > 1) us += 4.0 + 1e-3 * (double)rows * (0.35 + 0.16 * s * HD / 128);
+        if (s == 1 || us < best_us) {
+            best = s;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+// Causal attention of more query rows per kv head than one decode takes
+// (aw_multihead_attention_device): prefill_kernel over tiles of 128 rows.
+template <int HD>
+int launch_prefill(aw_engine* e, const aw_decode_desc* d, uint32_t n, uint32_t kv_len, hipStream_t st) {
+    aw::PrefillArgs a{};
+    a.q = d->q;
+    a.k = d->hot_k;
+    a.v = d->hot_v;
+    a.out = d->out;
+    a.n = n;
+    a.kv_len = kv_len;
+    a.q_heads = d->q_heads;
+    a.kv_heads = d->kv_heads;
+    a.gqa = d->q_heads / d->kv_heads;
+    a.rows = n * a.gqa;
+    a.tiles = cdiv(a.rows, (uint32_t)aw::kPrefillRows);
+    a.scale_log2 = d->scale * aw::kLog2e;
+    const uint64_t items = (uint64_t)a.tiles * a.kv_heads;
+    a.splits = prefill_splits(items, cdiv(kv_len, aw::kPrefillTokens), (uint64_t)a.kv_heads * a.rows, HD, e->n_cu);
+    const uint64_t part = (uint64_t)a.kv_heads * a.splits * a.rows;
+    const size_t stat = align_up(part * 4, kAlign), need = 2 * stat + part * HD * 4;
+    // A call being captured cannot grow the workspace: without parts it needs none.
+    if (a.splits > 1 && need > e->ws.cap && capturing(st)) a.splits = 1;
+    aw::MergeArgs m{};
+    if (a.splits > 1) {
+        const int rc = ensure_keep(e->ws, need, e->retired_ws, e->last_error, st);
+        if (rc) return rc;
+        char* ws = (char*)e->ws.ptr;
+        a.part_m = (float*)ws;
+        a.part_l = (float*)(ws + stat);
+        a.part_o = (float*)(ws + 2 * stat);
+    }
+    {
+        StageTimer t(e, AW_STAGE_HOT, st);
+        hipLaunchKernelGGL((aw::prefill_kernel<HD>), dim3((uint32_t)(items * a.splits)), dim3(aw::kPrefillThreads),
+                           aw::prefill_lds_bytes(HD), st, a);
+        AW_HIP(e, hipGetLastError());
+    }
+    if (a.splits == 1) return AW_OK;
+    m.hot_m = a.part_m;
+    m.hot_l = a.part_l;
+    m.hot_o = a.part_o;
+    m.out = a.out;
+    m.batch = 1;
+    m.queries = n;
+    m.q_heads = a.q_heads;
+    m.kv_heads = a.kv_heads;
+    m.gqa = a.gqa;
+    m.rows_r = a.rows;
+    m.hot_splits = a.splits;
+    m.total_rows = (uint64_t)a.kv_heads * a.rows;
+    return enqueue_merge<HD>(e, m, st);
 }
 
 template <typename F>
@@ -1134,6 +1221,8 @@ int aw_engine_create(int device, aw_engine** out) {
                               (const void*)aw::project_valu_kernel<128, kProjValuTa, kProjValuRb>,
                               (const void*)aw::project_valu_kernel<64, kProjValuTa, kProjValuRb>};
         for (const void* f : proj) set_lds(f);
+        set_lds((const void*)aw::prefill_kernel<64>);
+        set_lds((const void*)aw::prefill_kernel<128>);
         if (!aw_engine_internal::ops_set_lds_limits(e->max_lds)) attr_ok = false;
     }
     if (!attr_ok) {
@@ -1275,22 +1364,10 @@ int aw_multihead_attention_device(aw_engine* e, const uint16_t* q, const uint16_
     if (blocks > 0xFFFFFFFFull / kBlock) return fail(e, AW_E_UNSUPPORTED, "kv_len too large");
     AW_HIP(e, hipSetDevice(e->device));
     hipStream_t st = (hipStream_t)stream; // NULL is HIP's null stream
-    if (blocks > e->iota_n) {
-        // Grown (and kept, like the workspace) on the host's side: filled with a
-        // synchronous copy, so calls on any stream see it complete.
-        int rc = ensure_keep(e->iota, blocks * 4, e->retired_ws, e->last_error, st);
-        if (rc) return rc;
-        const uint32_t n = (uint32_t)std::min<size_t>(e->iota.cap / 4, 0xFFFFFFFFull);
-        std::vector<uint32_t> ids(n);
-        for (uint32_t i = 0; i < n; ++i) ids[i] = i;
-        AW_HIP(e, hipMemcpy(e->iota.ptr, ids.data(), (size_t)n * 4, hipMemcpyHostToDevice));
-        e->iota_n = n;
-    }
-    const uint32_t per = 64 / G; // queries of one call: G * queries <= 64 rows per kv head
+    const uint32_t per = 64 / G; // queries of one decode: G * queries <= 64 rows per kv head
     const size_t qrow = (size_t)q_heads * head_dim;
-    for (uint32_t j0 = 0; j0 < num_queries; j0 += per) {
-        const uint32_t c = std::min(per, num_queries - j0);
-        // The group's last query is token kv_len - num_queries + j0 + c - 1 of the cache.
+    // The decode of queries j0 .. j0 + c - 1; its last query is token kv_len - num_queries + j0 + c - 1 of the cache.
+    auto group = [&](uint32_t j0, uint32_t c) {
         const uint32_t n_tok = (uint32_t)((uint64_t)kv_len + j0 + c - num_queries);
         aw_decode_desc d{};
         d.layers = 1;
@@ -1308,8 +1385,35 @@ int aw_multihead_attention_device(aw_engine* e, const uint16_t* q, const uint16_
         d.q = q + j0 * qrow;
         d.hot_k = k_cache;
         d.hot_v = v_cache;
-        d.refs = (const uint32_t*)e->iota.ptr;
         d.out = out + j0 * qrow;
+        return d;
+    };
+    if (num_queries > per && (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15u) == 0 &&
+        (uint64_t)num_queries * G < (1u << 30) && (uint64_t)kv_heads * head_dim <= (1u << 16)) {
+        aw_decode_desc d = group((num_queries - 1) / per * per, (num_queries - 1) % per + 1);
+        Layout o;
+        char msg[256] = {0};
+        int rc = plan(&d, e->max_lds, e->n_cu, e->hot_wpc, e->cold_output, &o, msg, sizeof msg);
+        if (rc) return fail(e, rc, "%s", msg);
+        d.q = q;
+        d.out = out;
+        return head_dim == 64 ? launch_prefill<64>(e, &d, num_queries, kv_len, st)
+                              : launch_prefill<128>(e, &d, num_queries, kv_len, st);
+    }
+    if (blocks > e->iota_n) {
+        // Grown (and kept, like the workspace) on the host's side: filled with a
+        // synchronous copy, so calls on any stream see it complete.
+        int rc = ensure_keep(e->iota, blocks * 4, e->retired_ws, e->last_error, st);
+        if (rc) return rc;
+        const uint32_t n = (uint32_t)std::min<size_t>(e->iota.cap / 4, 0xFFFFFFFFull);
+        std::vector<uint32_t> ids(n);
+        for (uint32_t i = 0; i < n; ++i) ids[i] = i;
+        AW_HIP(e, hipMemcpy(e->iota.ptr, ids.data(), (size_t)n * 4, hipMemcpyHostToDevice));
+        e->iota_n = n;
+    }
+    for (uint32_t j0 = 0; j0 < num_queries; j0 += per) {
+        aw_decode_desc d = group(j0, std::min(per, num_queries - j0));
+        d.refs = (const uint32_t*)e->iota.ptr;
         const int rc = decode_device(e, &d, st);
         if (rc) return rc;
     }

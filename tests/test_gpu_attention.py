@@ -429,3 +429,71 @@ def test_weaver_kv_cache_background_distill(engine, stream):
     print(f"background distill: {in_flight} steps ran with the pass in flight", flush=True)
     assert in_flight >= 1 and a.distilling == 0 and a.cold_tokens == 32768 + 16
     assert (a.cold_tokens, a.hot_first) == (b1.cold_tokens, b1.hot_first)
+
+
+# More query rows per kv head than one decode takes: tiles of 128 rows, steps of 64
+# positions, the positions cut into parts where there are few rows.
+@pytest.mark.parametrize("nq,kv_len,hq,hkv,d", [
+    (17, 17, 32, 8, 128),     # 68 rows, the fewest at G = 4; a first step that is all limits
+    (32, 64, 32, 8, 128),     # one whole tile and one whole step
+    (33, 65, 32, 8, 128),     # one row group and one position more
+    (300, 299, 8, 2, 64),     # query 0 sees nothing
+    (10, 4000, 14, 2, 64),    # G = 7: one tile, many parts, a last step of 32
+    (130, 1531, 12, 2, 128),  # G = 6, a head's tiles and parts ragged
+    (65, 200, 4, 4, 64),      # G = 1
+    (2, 700, 64, 1, 128),     # G = 64: one query is a whole decode
+    (1024, 1024, 32, 8, 64),  # many tiles, one part
+])
+def test_prompt_attention_matches_oracle(engine, stream, nq, kv_len, hq, hkv, d):
+    cap = -(-kv_len // 16) * 16 + 16
+    q, k, v = cache_case(nq * 31 + kv_len, nq, kv_len, hq, hkv, d, cap)
+    qt, kt, vt = (torch.from_numpy(x.view(np.int16)).cuda() for x in (q, k, v))
+    print(f"attention: nq {nq} kv_len {kv_len} heads {hq}/{hkv} d {d}", flush=True)
+    engine.multihead_attention(qt, kt, vt, qt, kv_len, d, hq, hkv, nq, cache_tokens=cap, stream=stream)  # in place
+    engine.check_device_errors(stream)
+    assert_close(qt.view(torch.float16).double().cpu().numpy(),
+                 AO.multihead_attention_f64(q, k[:kv_len], v[:kv_len], kv_len, nq), (nq, kv_len))
+
+
+@pytest.mark.parametrize("nq,kv_len", [(100, 100), (40, 2000)])
+def test_prompt_attention_infinite_value(engine, stream, nq, kv_len):
+    """An inf and a NaN among the values reach the queries that see them and no other."""
+    hq, hkv, d = 8, 2, 128
+    cap = -(-kv_len // 16) * 16
+    q, k, v = cache_case(5, nq, kv_len, hq, hkv, d, cap)
+    ref = AO.multihead_attention_f64(q, k[:kv_len], v[:kv_len], kv_len, nq)
+    first = kv_len - nq + 21  # the position of query 21
+    v[first, 1, 5], v[first + 3, 1, 70] = np.inf, np.nan
+    qt, kt, vt = (torch.from_numpy(x.view(np.int16)).cuda() for x in (q, k, v))
+    out = torch.empty((nq, hq, d), dtype=torch.float16, device="cuda:0")
+    engine.multihead_attention(qt, kt, vt, out, kv_len, d, hq, hkv, nq, cache_tokens=cap, stream=stream)
+    engine.check_device_errors(stream)
+    got = out.double().cpu().numpy()
+    heads = slice(hq // 2, hq)  # kv head 1
+    assert np.isposinf(got[21:, heads, 5]).all() and np.isnan(got[24:, heads, 70]).all()
+    got[21:, heads, 5], got[24:, heads, 70] = ref[21:, heads, 5], ref[24:, heads, 70]
+    assert_close(got, ref)
+
+
+def test_prompt_attention_captured_without_workspace(stream):
+    """A first call that is captured: no workspace to put parts in, the same result on every replay."""
+    from aether_nexus_amd.weaver import WeaverEngine
+    nq, kv_len, hq, hkv, d = 33, 2000, 8, 2, 64
+    q, k, v = cache_case(9, nq, kv_len, hq, hkv, d, kv_len)
+    qt, kt, vt = (torch.from_numpy(x.view(np.int16)).cuda() for x in (q, k, v))
+    out = torch.empty((nq, hq, d), dtype=torch.float16, device="cuda:0")
+    with WeaverEngine() as eng:
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            eng.multihead_attention(qt, kt, vt, out, kv_len, d, hq, hkv, nq, cache_tokens=kv_len)
+        ref = AO.multihead_attention_f64(q, k, v, kv_len, nq)
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_close(out.double().cpu().numpy(), ref)
+        eager = torch.empty_like(out)
+        eng.multihead_attention(qt, kt, vt, eager, kv_len, d, hq, hkv, nq, cache_tokens=kv_len)
+        assert_close(eager.double().cpu().numpy(), ref)
+        torch.cuda.synchronize()
