@@ -9,9 +9,11 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <tuple>
 
 #include "../../include/aether_ops.h"
 #include "engine_internal.hpp"
+#include "gemm_kernels.hpp"
 #include "ops_kernels.hpp"
 
 namespace {
@@ -60,9 +62,56 @@ struct Product {
     uint32_t n;
 };
 
+// The tiles of a product of more than 64 rows.
+using GemmTiles = std::tuple<awo::GemmTile<4, 2, 4, 8, 2, 3>, awo::GemmTile<4, 2, 4, 5, 3>, awo::GemmTile<4, 2, 4, 4, 3>,
+                             awo::GemmTile<4, 2, 2, 4, 3>, awo::GemmTile<4, 2, 2, 2, 3>, awo::GemmTile<4, 2, 1, 3, 4>,
+                             awo::GemmTile<4, 2, 1, 2, 4>, awo::GemmTile<2, 2, 2, 1, 6>>;
+
+// f(T{}) for each tile.
+template <typename F>
+void each_tile(F f) {
+    std::apply([&](auto... t) { (f(t), ...); }, GemmTiles{});
+}
+
+// Tiles of all groups.
+template <typename T>
+uint64_t tile_count(const awo::GemmArgs& g) {
+    uint64_t n = 0;
+    for (uint32_t i = 0; i < g.groups; ++i) n += cdiv64(g.g[i].N, T::TN);
+    return n * cdiv64(g.M, T::TM);
+}
+
+// Estimated time (us) of a product on tile T, fitted to this GPU (M 72 .. 2048, N 896
+// .. 14336, K 896 .. 14336; the estimate's choice is within 10% of the fastest tile).
+// A 64-k stage takes a CU 2.2 ns per staged row (its loads, 58 bytes a ns), 1.9 with
+// two work-groups on it, or, with every CU busy, its products at 1.25 PFLOP/s (the
+// power limit); a tile starts and stores in 1.5 us and 15 halves a ns.  Measured, us:
+// 2048 x 14336 x 4096 256 x 256 tiles 222, 256 x 128 259; 2048 x 4096 x 14336 256 x
+// 128 217, 256 x 256 256; 512 x 4096 x 14336 128 x 64 95, 64 x 64 114, 128 x 128
+// 129; 117 x 3072 x 2048 64 x 32 8.3, 64 x 64 8.9, 128 x 64 11.3.
+template <typename T>
+double tile_us(const awo::GemmArgs& g, uint32_t n_cu) {
+    const uint64_t tiles = tile_count<T>(g), rounds = cdiv64(tiles, n_cu);
+    const double per_row = rounds > 1 && T::kLdsBytes <= 80 * 1024 ? 1.9e-3 : 2.2e-3;
+    const double area = (double)T::TM * T::TN, busy = (double)tiles / ((double)rounds * n_cu);
+    const double stage = std::max(per_row * (T::TM + T::TN), 2.6e-5 * area * busy);
+    return (double)rounds * ((double)cdiv64(g.K, awo::kStageK) * stage + 1.5 + area / 15e3);
+}
+
+template <typename T, bool F32, awo::Epi EPI>
+void launch_tile(const awo::GemmArgs& a, hipStream_t st) {
+    awo::GemmArgs g = a;
+    for (uint32_t i = 0; i < g.groups; ++i) {
+        g.g[i].tiles = (uint32_t)cdiv64(g.g[i].N, T::TN);
+        g.g[i].vec_out = g.g[i].N % 8 == 0 && aligned(g.g[i].C, 16);
+    }
+    hipLaunchKernelGGL((awo::gemm_tile_kernel<T, F32, EPI>), dim3((uint32_t)tile_count<T>(g)), dim3(T::kThreads),
+                       T::kLdsBytes, st, g);
+}
+
 // The products `p[0 .. np)` over the same activations a [m][k], one launch when
-// m <= 64 (skinny), one launch each otherwise (tiled).  EPI picks the store;
-// F32 the scaled fp32 output of matmul_scaled.
+// m <= 64 (skinny) or on gemm_tile_kernel, one launch each otherwise.  EPI picks the
+// store; F32 the scaled fp32 output of matmul_scaled.
 template <awo::Epi EPI, bool F32>
 int launch_products(aw_engine* e, const char* what, const uint16_t* a, const Product* p, int np, uint32_t m,
                     uint32_t k, float scale, hipStream_t st) {
@@ -93,28 +142,32 @@ int launch_products(aw_engine* e, const char* what, const uint16_t* a, const Pro
         if (EPI == awo::Epi::SiluGate)
             return ei::fail(e, AW_E_UNSUPPORTED, "%s: m = %u rows (the fused gate takes m <= 64; use matmul and "
                                                  "silu_gate)", what, m);
-        // One tiled launch per product, group 0 of its own arguments.
-        for (uint32_t i = 0; i < g.groups; ++i) {
-            awo::GemmArgs t = g;
-            t.g[0] = g.g[i];
-            t.groups = 1;
-            // 256 x 128 tiles when they fill the CUs at least once (16-byte rows, each
-            // operand below 4 GiB - 64 KiB for the buffer loads), else 128 x 128.
-            const dim3 wgrid((uint32_t)cdiv64(t.g[0].N, awo::kWideN), (uint32_t)cdiv64(m, awo::kWideM));
-            const uint64_t lim = (1ull << 32) - 65536;
-            const bool wide = vec && (uint64_t)wgrid.x * wgrid.y >= ei::compute_units(e) &&
-                              (uint64_t)t.g[0].N * k * 2 < lim && (uint64_t)m * k * 2 < lim;
-            const dim3 grid = wide ? wgrid : dim3((uint32_t)cdiv64(t.g[0].N, awo::kTileN), (uint32_t)cdiv64(m, awo::kTileM));
-            if (grid.y > 65535u) return ei::fail(e, AW_E_UNSUPPORTED, "%s: m = %u rows exceed the grid", what, m);
-            if constexpr (EPI != awo::Epi::SiluGate) {
-                if (wide && k % awo::kWideK != 0)
-                    hipLaunchKernelGGL((awo::gemm_wide_kernel<true, F32, EPI>), grid, dim3(awo::kWideThreads), awo::kWideLdsBytes, st, t);
-                else if (wide)
-                    hipLaunchKernelGGL((awo::gemm_wide_kernel<false, F32, EPI>), grid, dim3(awo::kWideThreads), awo::kWideLdsBytes, st, t);
-                else if (vec)
-                    hipLaunchKernelGGL((awo::gemm_tiled_kernel<true, F32, EPI>), grid, dim3(256), 0, st, t);
-                else
-                    hipLaunchKernelGGL((awo::gemm_tiled_kernel<false, F32, EPI>), grid, dim3(256), 0, st, t);
+        if (cdiv64(m, awo::kTileM) > 65535u)
+            return ei::fail(e, AW_E_UNSUPPORTED, "%s: m = %u rows exceed the grid", what, m);
+        if constexpr (EPI != awo::Epi::SiluGate) {
+            // 16-byte rows, a tile's rows below the buffer loads' limit.
+            if (vec && (uint64_t)k * 512 <= awo::kTileBytesMax) {
+                const uint32_t n_cu = ei::compute_units(e);
+                double best = 0.0;
+                void (*launch)(const awo::GemmArgs&, hipStream_t) = nullptr;
+                each_tile([&](auto t) {
+                    using T = decltype(t);
+                    const double us = tile_us<T>(g, n_cu);
+                    if (tile_count<T>(g) <= 0x7FFFFFFFull && (!launch || us < best)) {
+                        best = us;
+                        launch = launch_tile<T, F32, EPI>;
+                    }
+                });
+                if (!launch) return ei::fail(e, AW_E_UNSUPPORTED, "%s: grid too large", what);
+                launch(g, st);
+            } else {
+                for (uint32_t i = 0; i < g.groups; ++i) { // one launch per product, group 0 of its own arguments
+                    awo::GemmArgs t = g;
+                    t.g[0] = g.g[i];
+                    t.groups = 1;
+                    const dim3 grid((uint32_t)cdiv64(t.g[0].N, awo::kTileN), (uint32_t)cdiv64(m, awo::kTileM));
+                    hipLaunchKernelGGL((awo::gemm_tiled_kernel<F32, EPI>), grid, dim3(256), 0, st, t);
+                }
             }
         }
         OPS_HIP(e, hipGetLastError());
@@ -155,20 +208,21 @@ int launch_products(aw_engine* e, const char* what, const uint16_t* a, const Pro
 namespace aw_engine_internal {
 
 bool ops_set_lds_limits(size_t max_lds) {
-    // <MASK, F32, EPI> of the products that take the wide tiles.
-    const void* fns[] = {(const void*)awo::gemm_wide_kernel<true, false, awo::Epi::Store>,
-                         (const void*)awo::gemm_wide_kernel<false, false, awo::Epi::Store>,
-                         (const void*)awo::gemm_wide_kernel<true, true, awo::Epi::Store>,
-                         (const void*)awo::gemm_wide_kernel<false, true, awo::Epi::Store>,
-                         (const void*)awo::gemm_wide_kernel<true, false, awo::Epi::Residual>,
-                         (const void*)awo::gemm_wide_kernel<false, false, awo::Epi::Residual>};
     bool ok = true;
-    for (const void* f : fns)
+    auto set = [&](const void* f) {
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds) != hipSuccess) {
             ok = false;
             (void)hipGetLastError();
         }
-    return ok && max_lds >= awo::kWideLdsBytes;
+    };
+    each_tile([&](auto t) {
+        using T = decltype(t);
+        ok = ok && max_lds >= T::kLdsBytes;
+        set((const void*)awo::gemm_tile_kernel<T, false, awo::Epi::Store>);
+        set((const void*)awo::gemm_tile_kernel<T, true, awo::Epi::Store>);
+        set((const void*)awo::gemm_tile_kernel<T, false, awo::Epi::Residual>);
+    });
+    return ok;
 }
 
 } // namespace aw_engine_internal

@@ -308,9 +308,8 @@ def test_fused_products_match_the_separate_calls(ops, m):
 
 @pytest.mark.parametrize("k", [520, 517])
 def test_wide_and_tiled_products_same_bits(ops, k):
-    """Products with many 256 x 128 tiles take gemm_wide_kernel (K % 8 == 0),
-    smaller ones the 128 x 128 tiles; both sum the same k-steps of 32 in the same
-    order, so the columns a small product shares with a large one have the same
+    """Large products take 256-row tiles of gemm_tile_kernel (K % 8 == 0), smaller
+    ones its 64-row tiles; all sum the same k-steps of 32 in the same order, so the columns a small product shares with a large one have the same
     bits, for the f16 store, the residual form and the scaled fp32 store (K = 520:
     a partial last k-step; K = 517: both on the 128 x 128 tiles)."""
     import torch
@@ -333,6 +332,43 @@ def test_wide_and_tiled_products_same_bits(ops, k):
     ops.matmul_scaled(a, bb, fb, m, n, k, 0.25)
     ops.matmul_scaled(a, bs, fs, m, ns, k, 0.25)
     assert torch.equal(fb[:, :ns].contiguous().view(torch.int32), fs.view(torch.int32)), "scaled"
+
+
+# A shape that takes each tile of gemm_tile_kernel (256 x 256, 256 x 160, 256 x 128, 128 x 128,
+# 128 x 64, 64 x 96, 64 x 64, 64 x 32), ragged in M and N (8-wide stores and not), with one stage of
+# K, a partial one, fewer than the tile's LDS buffers and more.
+TILE_SHAPES = [(2000, 8008, 200), (1000, 8200, 520), (500, 14001, 72), (700, 5000, 72), (200, 8190, 136),
+               (300, 4868, 128), (300, 2056, 1032), (65, 96, 264), (129, 1, 8), (66, 33, 64), (8400, 40, 24)]
+
+
+@pytest.mark.parametrize("m,n,k", TILE_SHAPES, ids=[f"{m}x{n}x{k}" for m, n, k in TILE_SHAPES])
+def test_tiles_match_the_gathered_loads(ops, m, n, k):
+    """Activations two bytes past a 16-byte boundary take the kernel that gathers its
+    operands element by element, in the same order of sums: the same bits from
+    every tile, for the store, the residual form, the scaled fp32 store and q/k/v."""
+    import torch
+    print(f"tiles {m}x{n}x{k}", flush=True)
+    g = torch.Generator(device="cuda:0").manual_seed(m + n + k)
+
+    def rand(*shape, scale=1.0):
+        return (torch.randn(shape, generator=g, device="cuda:0") * scale).to(torch.float16)
+    a, b, x0 = rand(m, k), rand(n, k, scale=0.1), rand(m, n)
+    off = torch.empty(m * k + 1, dtype=torch.float16, device="cuda:0")[1:].view(m, k)
+    off.copy_(a)
+    got = []
+    for x in (a, off):
+        out, res = torch.full((m, n), float("nan"), dtype=torch.float16, device="cuda:0"), x0.clone()
+        f32 = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda:0")
+        qkv = [torch.full((m, w), float("nan"), dtype=torch.float16, device="cuda:0") for w in (n, n // 2 + 1, n // 2 + 1)]
+        ops.matmul(x, b, out, m, n, k)
+        ops.matmul_add_residual(x, b, res, m, n, k, 0.5)
+        ops.matmul_scaled(x, b, f32, m, n, k, 0.25)
+        ops.matmul_qkv(x, b, b, b[n - n // 2 - 1:], *qkv, m, n, n // 2 + 1, k)
+        got.append([out, res, f32, *qkv])
+    for i, (t, w) in enumerate(zip(*got)):
+        assert bool(torch.isfinite(t).all()) and torch.equal(t, w), i
+    rows = torch.unique(torch.cat([torch.arange(min(m, 16)), torch.tensor([m // 2, m - 1])]))
+    check_product(host(got[0][0])[rows], host(a)[rows], host(b), k, f"tiles {m}x{n}x{k}")
 
 
 def test_product_bits_do_not_depend_on_the_wave_count(ops):
