@@ -40,7 +40,7 @@ from typing import Callable, Optional, Sequence
 import numpy as np
 import torch
 
-from .weaver import make_desc, make_encode_desc
+from .weaver import current_raw_stream, make_desc, make_encode_desc
 
 MAX_SEQ_LEN = 4096  # InferenceEngine::MAX_SEQ_LEN (inference.rs:219)
 MAX_BATCH = 16  # InferenceEngine::MAX_BATCH (inference.rs:221): tokens per forward_batch
@@ -51,12 +51,16 @@ def _torch_stream(handle: Optional[int]):
     """torch's Stream object for a hipStream_t handle: torch's current stream for
     None or its handle, the null stream for 0 (torch.cuda.ExternalStream(0) makes
     a stream of its own instead), else an external stream wrapping the handle."""
-    cur = torch.cuda.current_stream()
-    if handle is None or handle == cur.cuda_stream:
-        return cur
+    if handle is None or handle == current_raw_stream(torch):
+        return torch.cuda.current_stream()
     if handle == 0:
         return torch.cuda.default_stream()
     return torch.cuda.ExternalStream(handle)
+
+
+def _is_current(s) -> bool:
+    """Whether torch's current stream is `s` (entering it again would cost 10 us)."""
+    return s.cuda_stream == current_raw_stream(torch) and s.device_index == torch._C._cuda_getDevice()
 
 
 class KvCacheError(RuntimeError):
@@ -207,6 +211,8 @@ class WeaverKvCache:
         None for a cache in host memory (the host-logic tests)."""
         if not self._cuda:
             return None
+        if stream is None and self._last is not None and _is_current(self._last):
+            return self._last  # the usual call, without a Stream object of its own
         s = _torch_stream(stream)
         if self._last is not None and self._last.cuda_stream != s.cuda_stream:
             with torch.cuda.stream(s):
@@ -221,7 +227,7 @@ class WeaverKvCache:
     @staticmethod
     def _on(s):
         """Torch work inside runs on stream `s` (none: as it is)."""
-        return torch.cuda.stream(s) if s is not None else contextlib.nullcontext()
+        return contextlib.nullcontext() if s is None or _is_current(s) else torch.cuda.stream(s)
 
     @staticmethod
     def _handle(s, stream: Optional[int]) -> Optional[int]:
@@ -257,8 +263,9 @@ class WeaverKvCache:
         while i < n:  # block by block (the ring may wrap)
             slot, off = self._slot(t + i)
             m = min(BLOCK_TOKENS - off, n - i)
-            self.k[layer][slot, off:off + m].copy_(k[i:i + m])
-            self.v[layer][slot, off:off + m].copy_(v[i:i + m])
+            ki, vi = (k, v) if m == n else (k[i:i + m], v[i:i + m])
+            self.k[layer][slot, off:off + m].copy_(ki)
+            self.v[layer][slot, off:off + m].copy_(vi)
             i += m
 
     def refs(self, hot_blocks: int) -> torch.Tensor:
@@ -302,8 +309,10 @@ class WeaverKvCache:
             raise KvCacheError("q and out must be [num_tokens][q_heads][head_dim], q_heads a multiple of kv_heads")
         hot_tok = self.hot_tokens(self.position + n)
         hot_blocks = -(-hot_tok // BLOCK_TOKENS)
-        with self._on(s):
-            refs = self.refs(hot_blocks)
+        refs = self._refs
+        if self._refs_key != (self.hot_first, hot_blocks, self.cold_blocks):
+            with self._on(s):
+                refs = self.refs(hot_blocks)
         desc = make_desc(layers=1, batch=1, queries=n, q_heads=q_heads, kv_heads=self.kv_heads, head_dim=head_dim,
                          dict_size=self.dict_size, dict_heads=self.dict_heads, hot_count=hot_blocks,
                          cold_count=self.cold_blocks, refs_stride=max(hot_blocks + self.cold_blocks, 1),
