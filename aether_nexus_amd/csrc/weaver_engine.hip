@@ -1221,6 +1221,8 @@ int aw_engine_create(int device, aw_engine** out) {
                               (const void*)aw::project_valu_kernel<128, kProjValuTa, kProjValuRb>,
                               (const void*)aw::project_valu_kernel<64, kProjValuTa, kProjValuRb>};
         for (const void* f : proj) set_lds(f);
+        set_lds((const void*)aw::encode_lds_kernel<64>);
+        set_lds((const void*)aw::encode_lds_kernel<128>);
         set_lds((const void*)aw::prefill_kernel<64>);
         set_lds((const void*)aw::prefill_kernel<128>);
         if (!aw_engine_internal::ops_set_lds_limits(e->max_lds)) attr_ok = false;
@@ -1512,13 +1514,15 @@ int encode_device(aw_engine* e, const aw_encode_desc* d, hipStream_t st) {
     // Scratch of the MFMA path (the atoms' norms), allocated before any work is queued.
     const bool full_scan = (d->flags & AW_F_ENCODE_FULL_SCAN) != 0;
     const uint64_t n_atoms = (uint64_t)d->dict_heads * d->dict_size;
-    if (!full_scan && (rc = ensure_keep(e->enc_ws, n_atoms * sizeof(aw::AtomNorm), e->retired_ws, e->last_error, st)))
+    const size_t enc_lds = aw::enc_lds_bytes(d->dict_size, d->head_dim);
+    const bool resident = !full_scan && (uint64_t)d->dict_size * d->head_dim * 2 <= aw::kEncLdsDict && enc_lds <= e->max_lds;
+    if (!full_scan && !resident && (rc = ensure_keep(e->enc_ws, n_atoms * sizeof(aw::AtomNorm), e->retired_ws, e->last_error, st)))
         return rc;
     // The entropy proxy (few long lanes) runs on the side stream beside the encoder.
     if (d->entropy) {
         AW_HIP(e, hipEventRecord(e->ev_fork, st));
         AW_HIP(e, hipStreamWaitEvent(e->side, e->ev_fork, 0));
-        hipLaunchKernelGGL(aw::entropy_kernel, dim3(cdiv(d->n_blocks, aw::kEntBlocks)), dim3(64), 0, e->side, a, d->head_dim);
+        hipLaunchKernelGGL(aw::entropy_kernel, dim3(cdiv(d->n_blocks, aw::kEntBlocks)), dim3(aw::kEntThreads), 0, e->side, a, d->head_dim);
         AW_HIP(e, hipGetLastError());
         AW_HIP(e, hipEventRecord(e->ev_join, e->side));
     }
@@ -1528,6 +1532,15 @@ int encode_device(aw_engine* e, const aw_encode_desc* d, hipStream_t st) {
             hipLaunchKernelGGL(aw::encode_kernel<64>, grid, dim3(aw::kEncThreads), 0, st, a);
         else
             hipLaunchKernelGGL(aw::encode_kernel<128>, grid, dim3(aw::kEncThreads), 0, st, a);
+    } else if (resident) {
+        // Dictionaries that fit in LDS (512 atoms of 128 dims).  A CU per work-group (its
+        // LDS), shared out over the heads; a wave per 64 tokens.
+        const uint32_t wgs = std::max(1u, std::min(e->n_cu / d->kv_heads, (uint32_t)cdiv((uint64_t)d->n_blocks * kBlock, 64)));
+        const dim3 grid(wgs * d->kv_heads);
+        if (d->head_dim == 64)
+            hipLaunchKernelGGL(aw::encode_lds_kernel<64>, grid, dim3(aw::kEncLThreads), enc_lds, st, a, wgs);
+        else
+            hipLaunchKernelGGL(aw::encode_lds_kernel<128>, grid, dim3(aw::kEncLThreads), enc_lds, st, a, wgs);
     } else {
         // MFMA prefilter + exact rescoring: the atoms' norms first.
         aw::AtomNorm* dn = (aw::AtomNorm*)e->enc_ws.ptr;
@@ -1571,8 +1584,8 @@ int aw_block_entropy_device(aw_engine* e, const uint16_t* hot, uint64_t hot_bloc
     a.kv_heads = kv_heads;
     a.n_blocks = n_blocks;
     a.hot_blocks = hot_blocks;
-    hipLaunchKernelGGL(aw::entropy_kernel, dim3(cdiv(n_blocks, aw::kEntBlocks)), dim3(64), 0, (hipStream_t)stream, a,
-                       head_dim);
+    hipLaunchKernelGGL(aw::entropy_kernel, dim3(cdiv(n_blocks, aw::kEntBlocks)), dim3(aw::kEntThreads), 0,
+                       (hipStream_t)stream, a, head_dim);
     AW_HIP(e, hipGetLastError());
     return AW_OK;
 }

@@ -2678,6 +2678,7 @@ constexpr int kEncMSub = kEncMCap / 4; // per token and lane: each of 4 lanes se
 constexpr uint32_t kDictBad = 1u, kDictSubnormal = 2u;
 
 typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef double double2_t __attribute__((ext_vector_type(2)));
 
 // |d_a|_2 and |d_a|_1 (rounded up) and flags (kDictBad: inf or NaN component;
 // kDictSubnormal) for every atom of every dictionary head, as {l2, l1, flags}.
@@ -2997,179 +2998,559 @@ __global__ __launch_bounds__(kEncMThreads) void encode_mfma_kernel(EncodeArgs a,
     a.cold[(uint64_t)c * kBlockTokens * a.kv_heads + tt3 * a.s_tok + g * a.s_head] = code;
 }
 
-// Variance proxy of each listed block (distiller.rs:126-159), bit-exact: one
-// lane per block runs the reference's loops in memory order, in f64, with no
-// fused multiply-add (the reference squares, then adds), and returns f32; an
-// all-zero block gives 0.  Without a block list (src null) lane i takes block i.
+// ------------------------------------- encoder: the dictionary resident in LDS
 //
-// The f64 sums are sequential chains, so a block cannot be split across lanes;
-// what is parallel is the data supply.  One wave owns kEntBlocks blocks and
-// streams them in chunks of kEntChunk values: the wave loads a chunk of all its
-// blocks with coalesced 16-byte loads (16 lanes per 256-byte block chunk) into
-// one of two LDS tiles while each block's lane runs its chain over the other
-// tile.  Rows are padded by 16 bytes so the lanes' row reads spread over the
-// banks.
-constexpr int kEntChunk = 128;                   // f16 values per block and chunk (256 bytes)
-constexpr int kEntCols = kEntChunk / 8;          // 16-byte words per row
-constexpr int kEntPitch = kEntCols + 1;          // padded row, in 16-byte words
+// The codes of encode_kernel (bit for bit) in one MFMA pass, for dictionaries of
+// at most kEncLdsDict bytes per head.  Work-group = 8 waves of one kv head with the
+// head's dictionary in LDS; a wave takes tiles of 64 tokens, without barriers.  As in
+// encode_mfma_kernel |M_a - S_a| <= E, here one E per token from the head's largest
+// norms (good atoms).  Lane (token li, lg) sees a quarter of the atoms and keeps its 5
+// largest scores, each packed with the atom's number in the low NB bits of the float:
+// p with |p - M| < 2^(NB-23) |p|.  With slack(p) = E + 2^(NB-22) |p|:
+//   P4 = the 4th largest p of the token's four lanes, T = P4 - slack(P4): four atoms
+//   have S >= T, so only atoms with p + slack(p) >= T can reach the top 4;
+//   a lane whose 5th p reaches T may have dropped such an atom, and a score too small
+//   to carry the number (denormal) may have lost it: those tokens, and those with an
+//   inf or NaN component, are scanned exactly, their atoms over the wave's lanes.
+// The candidates (4.03 a token on average) are rescored exactly, lane = token, from
+// the dictionary in LDS; the insertion orders by (score desc, atom asc), so the
+// order of the candidates does not matter.  Atoms with an inf or NaN component stay
+// out of the bound and are always rescored.
+// Dictionary rows are HD / 8 16-byte chunks, chunk c of row r at c ^ (r % chunks): the
+// fragment reads (16 rows, one chunk) meet no bank conflict, and the rescoring's
+// random rows spread over the banks.
+// Bound: the vector ALUs, 6 operations a score (pack, max, 4 medians; 169 of 332 us for
+// 8192 blocks of 8 heads x 128 dims, 512 atoms: loads 57, lists 38, rescoring 80; beside
+// that, two candidates rescored at once or the next tile's loads ahead of the
+// rescoring cost registers and were slower).  encode_mfma_kernel at the same size 587.
+constexpr int kEncLWaves = 8, kEncLThreads = 64 * kEncLWaves;
+constexpr size_t kEncLdsDict = 128 * 1024; // dictionary bytes of one head
+constexpr int kEncLRow = 12;               // list of a token: header (count, or kEncLFull), candidates
+constexpr uint32_t kEncLFull = 0xFFFFu;
+constexpr size_t enc_lds_bytes(uint32_t A, int HD) {
+    return (size_t)A * HD * 2 + (size_t)kEncLWaves * 64 * kEncLRow * 2 + 4 * 4 + 32 * 4;
+}
+
+template <int HD>
+__global__ __launch_bounds__(kEncLThreads) void encode_lds_kernel(EncodeArgs a, uint32_t wgs) {
+    constexpr int KS = HD / 32, PR = HD / 8, NTT = 4, NB = HD == 128 ? 7 : 8, ROW = kEncLRow;
+    extern __shared__ __attribute__((aligned(16))) unsigned char enc_lds[];
+    const uint32_t A = a.dict_size;
+    uint4_t* sd = (uint4_t*)enc_lds;                             // [A][PR], swizzled
+    uint16_t* lists = (uint16_t*)(enc_lds + (size_t)A * HD * 2); // [waves][64][ROW]
+    uint32_t* stat = (uint32_t*)(lists + kEncLWaves * 64 * ROW); // largest |d|_2, |d|_1 (float bits), flags
+    uint32_t* bad = stat + 4;                                    // [32] bit mask of the atoms with an inf or NaN
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t g = blockIdx.x % a.kv_heads, part = blockIdx.x / a.kv_heads;
+    const uint32_t n_tok = a.n_blocks * kBlockTokens;
+    const uint4_t* Dg = (const uint4_t*)(a.dict + (uint64_t)(a.dict_heads == 1 ? 0u : g) * A * HD);
+    constexpr float kBound = 8.0f * HD * 5.9604645e-8f; // 8 * HD * 2^-24
+    constexpr float kSub = 6.1035156e-5f;               // 2^-14: bound of a subnormal f16
+
+    for (uint32_t p = tid; p < A * PR; p += kEncLThreads) {
+        const uint32_t r = p / PR, c = p % PR;
+        sd[r * PR + (c ^ (r & (PR - 1)))] = Dg[p];
+    }
+    if (tid < 36) stat[tid] = 0u; // stat[4] and bad[32]
+    __syncthreads();
+    auto row_chunk = [&](uint32_t r, uint32_t c) { return sd[r * PR + (c ^ (r & (PR - 1)))]; };
+    for (uint32_t r = tid; r < A; r += kEncLThreads) {
+        float ss = 0.0f, s1 = 0.0f;
+        uint32_t fl = 0;
+        for (int j = 0; j < PR; ++j) {
+            const uint4_t w = row_chunk(r, j);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t bits = (w[e / 2] >> (16 * (e % 2))) & 0xFFFFu;
+                const uint32_t ex = (bits >> 10) & 31u, man = bits & 1023u;
+                fl |= ex == 31u ? kDictBad : 0u;
+                fl |= (ex == 0u && man != 0u) ? kDictSubnormal : 0u;
+                const float f = h2f_bits(bits);
+                ss = fmaf(f, f, ss);
+                s1 += fabsf(f);
+            }
+        }
+        if (fl & kDictBad) {
+            atomicOr(&bad[r / 32], 1u << (r & 31u));
+            atomicOr(&stat[2], kDictBad);
+        } else {
+            atomicMax(&stat[0], __builtin_bit_cast(uint32_t, sqrtf(ss) * 1.001f));
+            atomicMax(&stat[1], __builtin_bit_cast(uint32_t, s1 * 1.001f));
+            if (fl) atomicOr(&stat[2], kDictSubnormal);
+        }
+    }
+    __syncthreads();
+    const float l2m = __builtin_bit_cast(float, stat[0]), l1m = __builtin_bit_cast(float, stat[1]);
+    const uint32_t dfl = (uint32_t)__builtin_amdgcn_readfirstlane((int)stat[2]);
+    uint16_t* lst = lists + wave * 64 * ROW;
+    uint32_t keep = ~((1u << NB) - 1u);
+    __asm__("" : "+v"(keep)); // one v_bfi_b32 a score packs the atom's number
+
+    for (uint32_t wt = (uint32_t)wave * wgs + part; wt * 64u < n_tok; wt += (uint32_t)kEncLWaves * wgs) {
+        const uint32_t tok0 = wt * 64u;
+        half8_t xb[NTT][KS]; // the tile's tokens (B operands)
+        float E[NTT];
+        // Bit tt: a component of the lane's token tt is inf or NaN; all are zeros (then every
+        // score is, and the first four atoms are the code).
+        uint32_t xfl = 0, xzero = 0;
+#pragma unroll
+        for (int tt = 0; tt < NTT; ++tt) {
+            const uint32_t T = min(tok0 + (uint32_t)(tt * 16 + li), n_tok - 1u);
+            uint32_t b = a.src[T / kBlockTokens] & kRefMask;
+            b = b < a.hot_blocks ? b : 0u; // such a token is not written
+            const uint16_t* xp = a.hot + (((uint64_t)b * kBlockTokens + T % kBlockTokens) * a.kv_heads + g) * HD;
+            float ss = 0.0f, s1 = 0.0f;
+            ushort2_t lo = (ushort2_t)(uint16_t)0xFFFFu, hi = (ushort2_t)(uint16_t)0u; // of |x|'s bits: least - 1, largest
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const uint4_t w = *(const uint4_t*)(xp + 32 * ks + 8 * lg);
+                xb[tt][ks] = as_h8(w);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t wv = w[e], wa = wv & 0x7FFF7FFFu;
+                    const ushort2_t m = __builtin_bit_cast(ushort2_t, wa);
+                    ss = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, wv), __builtin_bit_cast(half2_t, wv), ss, false);
+                    s1 = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, wa), (half2_t)(_Float16)1.0f, s1, false);
+                    lo = __builtin_elementwise_min(lo, (ushort2_t)(m - (uint16_t)1u)); // a zero wraps to the top
+                    hi = __builtin_elementwise_max(hi, m);
+                }
+            }
+            const uint16_t least = lo[0] < lo[1] ? lo[0] : lo[1], most = hi[0] > hi[1] ? hi[0] : hi[1];
+            uint32_t fl = (least < 0x03FFu ? 2u : 0u) | (most >= 0x7C00u ? 1u : 0u) | (most ? 4u : 0u);
+            ss += __shfl_xor(ss, 16);
+            ss += __shfl_xor(ss, 32);
+            s1 += __shfl_xor(s1, 16);
+            s1 += __shfl_xor(s1, 32);
+            fl |= __shfl_xor(fl, 16);
+            fl |= __shfl_xor(fl, 32);
+            E[tt] = fmaf(kBound * (sqrtf(ss) * 1.001f), l2m,
+                         fmaf((fl & 2u) ? kSub : 0.0f, l1m, (dfl & kDictSubnormal) ? kSub * (s1 * 1.001f) : 0.0f));
+            E[tt] = E[tt] * 1.01f + 1e-36f; // the comparisons' own roundings
+            xfl |= (fl & 1u) << tt;
+            xzero |= (fl & 4u) || (dfl & kDictBad) ? 0u : 1u << tt;
+        }
+
+        float top[NTT][5];
+#pragma unroll
+        for (int tt = 0; tt < NTT; ++tt)
+#pragma unroll
+            for (int k = 0; k < 5; ++k) top[tt][k] = -INFINITY;
+        // All atoms; MASK: some of the head's have an inf or NaN.
+        auto scan = [&](auto mask_bad) {
+            constexpr bool MASK = decltype(mask_bad)::value;
+            const uint32_t tiles = A / 16u;
+            half8_t ad[KS];
+            auto fetch = [&](uint32_t at, int ks) {
+                ad[ks] = as_h8(row_chunk(min(at, tiles - 1u) * 16u + (uint32_t)li, (uint32_t)(4 * ks + lg)));
+            };
+            auto insert5 = [&](float sc, uint32_t id, bool is_bad, float(&t)[5]) {
+                uint32_t pb = (__builtin_bit_cast(uint32_t, sc) & keep) | (id & ~keep);
+                if constexpr (MASK) pb = is_bad ? 0xFF800000u : pb;
+                const float y = __builtin_bit_cast(float, pb);
+                float t0;
+                __asm__("v_max_f32 %0, %1, %2" : "=v"(t0) : "v"(t[0]), "v"(y)); // fmaxf quiets both operands first
+                const float t1 = __builtin_amdgcn_fmed3f(t[0], t[1], y);
+                const float t2 = __builtin_amdgcn_fmed3f(t[1], t[2], y);
+                const float t3 = __builtin_amdgcn_fmed3f(t[2], t[3], y);
+                t[4] = __builtin_amdgcn_fmed3f(t[3], t[4], y);
+                t[0] = t0;
+                t[1] = t1;
+                t[2] = t2;
+                t[3] = t3;
+            };
+            // Tile at's scores are inserted between the products of tile at + 1, whose
+            // fragments are in `ad`, and tile at + 2's are read.
+            auto step = [&](const float4_t(&cur)[NTT], float4_t(&next)[NTT], uint32_t at) {
+                uint32_t m = 0;
+                if constexpr (MASK) m = bad[at / 2u] >> (16u * (at & 1u) + 4u * (uint32_t)lg);
+                constexpr int PER = 16 / KS; // scores between the products of one k-step
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+                    for (int i = 0; i < PER; ++i) {
+                        const int q = ks * PER + i, tt = q / 4, e = q % 4;
+                        if (i % (PER / NTT) == 0) {
+                            const int nt = i / (PER / NTT);
+                            next[nt] = mfma16x16x32(ad[ks], xb[nt][ks], ks == 0 ? (float4_t)0.0f : next[nt]);
+                        }
+                        insert5(cur[tt][e], at * 4u + (uint32_t)e, (m >> e) & 1u, top[tt]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    fetch(at + 2u, ks);
+                }
+            };
+            float4_t acc0[NTT], acc1[NTT];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) fetch(0, ks);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int tt = 0; tt < NTT; ++tt)
+                    acc0[tt] = mfma16x16x32(ad[ks], xb[tt][ks], ks == 0 ? (float4_t)0.0f : acc0[tt]);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) fetch(1, ks);
+            for (uint32_t at = 0; at < tiles; at += 2u) {
+                step(acc0, acc1, at);
+                if (at + 1u < tiles) step(acc1, acc0, at + 1u);
+            }
+        };
+        if (dfl & kDictBad) scan(std::true_type{});
+        else scan(std::false_type{});
+
+        // Candidates into the token's list, the four lanes' one after another.
+#pragma unroll
+        for (int tt = 0; tt < NTT; ++tt) {
+            float t4[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) t4[k] = top[tt][k];
+#pragma unroll
+            for (int o = 16; o < 64; o *= 2) {
+                float y[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) y[k] = __shfl_xor(t4[k], o);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float n0 = fmaxf(t4[0], y[k]), n1 = __builtin_amdgcn_fmed3f(t4[0], t4[1], y[k]),
+                                n2 = __builtin_amdgcn_fmed3f(t4[1], t4[2], y[k]);
+                    t4[3] = __builtin_amdgcn_fmed3f(t4[2], t4[3], y[k]);
+                    t4[0] = n0;
+                    t4[1] = n1;
+                    t4[2] = n2;
+                }
+            }
+            constexpr float kPack = 1.0f / (float)(1u << (22 - NB));
+            const float thr = t4[3] - fmaf(fabsf(t4[3]), kPack, E[tt]);
+            uint32_t n = 0, full = (xfl >> tt) & 1u;
+            full |= t4[3] == -INFINITY ? 1u : 0u; // fewer than 4 good atoms
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                const float p = top[tt][k];
+                if (p + fmaf(fabsf(p), kPack, E[tt]) >= thr) {
+                    ++n;
+                    full |= (k == 4 || fabsf(p) < 1e-37f) ? 1u : 0u;
+                }
+            }
+            const bool zero = (xzero >> tt) & 1u;
+            if (zero) {
+                n = lg == 0 ? 4u : 0u;
+                full = 0u;
+            }
+            uint32_t off = 0, sum = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t v = (uint32_t)__shfl((int)(n | (full << 8)), li + 16 * q);
+                off += q < lg ? v & 255u : 0u;
+                sum += v;
+            }
+            const bool all = sum >= 256u || (sum & 255u) > (uint32_t)(ROW - 1);
+            uint16_t* tl = lst + (tt * 16 + li) * ROW;
+            if (lg == 0) tl[0] = (uint16_t)(all ? kEncLFull : sum);
+            if (!all) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t v = __builtin_bit_cast(uint32_t, top[tt][k]) & ((1u << NB) - 1u);
+                    if ((uint32_t)k < n) tl[1 + off + k] = (uint16_t)(zero ? (uint32_t)k : (v >> 2) * 16u + 4u * (uint32_t)lg + (v & 3u));
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); // the lists are the wave's own
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+        // Exact scores: lane = token.
+        const uint32_t T3 = tok0 + (uint32_t)lane;
+        const bool live = T3 < n_tok;
+        const uint32_t Tc = live ? T3 : n_tok - 1u, bi = Tc / kBlockTokens, tt3 = Tc % kBlockTokens;
+        const uint32_t b = a.src[bi] & kRefMask;
+        const uint32_t c = a.dst ? (a.dst[bi] & kRefMask) : b;
+        const bool ok = live && b < a.hot_blocks && c < a.cold_blocks;
+        if (live && g == 0 && tt3 == 0) { // one report per block
+            if (b >= a.hot_blocks) flag_error(a.err, kErrHotRef);
+            if (c >= a.cold_blocks) flag_error(a.err, kErrColdRef);
+        }
+        const uint64_t xat = (((uint64_t)(b < a.hot_blocks ? b : 0u) * kBlockTokens + tt3) * a.kv_heads + g) * HD;
+        const uint32_t n = lst[lane * ROW];
+        float v[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        uint32_t ix[4] = {0u, 0u, 0u, 0u};
+        // (s, ai) into the four best by (score desc, atom asc); NaN and -inf never enter.
+        auto insert = [&](float s, uint32_t ai) {
+            auto before = [&](int k) { return s > v[k] || (s == v[k] && ai < ix[k]); };
+            if (before(3)) {
+                const bool g0 = before(0), g1 = before(1), g2 = before(2);
+                v[3] = g2 ? v[2] : s;
+                ix[3] = g2 ? ix[2] : ai;
+                v[2] = g1 ? v[1] : (g2 ? s : v[2]);
+                ix[2] = g1 ? ix[1] : (g2 ? ai : ix[2]);
+                v[1] = g0 ? v[0] : (g1 ? s : v[1]);
+                ix[1] = g0 ? ix[0] : (g1 ? ai : ix[1]);
+                v[0] = g0 ? s : v[0];
+                ix[0] = g0 ? ai : ix[0];
+            }
+        };
+        half8_t x[PR];
+        auto load_x = [&](uint64_t at) {
+#pragma unroll
+            for (int j = 0; j < PR; ++j) x[j] = as_h8(*(const uint4_t*)(a.hot + at + 8 * j));
+        };
+        auto score = [&](uint32_t ai) {
+            float s = -0.0f;
+#pragma unroll
+            for (int j = 0; j < PR; ++j) {
+                const half8_t d8 = as_h8(row_chunk(ai, (uint32_t)j));
+                __asm__("" : "+v"(x[j])); // stays in halves: converted once, it would take twice the registers
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s = fmaf((float)x[j][e], (float)d8[e], s);
+            }
+            insert(s, ai);
+        };
+        load_x(xat);
+        const bool full = n == kEncLFull;
+        for (uint32_t i = 0; !full && i < n; ++i) score(lst[lane * ROW + 1 + i]);
+        if (dfl & kDictBad)
+            for (uint32_t ai = 0; ai < A; ++ai)
+                if ((bad[ai / 32u] >> (ai & 31u)) & 1u) // uniform
+                    if (!full) score(ai);
+        // Tokens scanned whole, one after another: lane l scores atoms l, l + 64, ..
+        for (uint64_t todo = __ballot(full && ok); todo; todo &= todo - 1u) {
+            const int t = __builtin_ctzll(todo);
+            float kv[4];
+            uint32_t kx[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { // this lane's own token aside
+                kv[k] = v[k];
+                kx[k] = ix[k];
+                v[k] = -INFINITY;
+                ix[k] = 0u;
+            }
+            load_x((uint64_t)__shfl((unsigned long long)xat, t));
+            for (uint32_t ai = (uint32_t)lane; ai < A; ai += 64u) score(ai);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { // the k-th best over the lanes; its lane drops it
+                float bv = v[0];
+                uint32_t bx = v[0] == -INFINITY ? 0xFFFFFFFFu : ix[0];
+#pragma unroll
+                for (int o = 1; o < 64; o *= 2) {
+                    const float ov = __shfl_xor(bv, o);
+                    const uint32_t ox = (uint32_t)__shfl_xor((int)bx, o);
+                    const bool take = ov > bv || (ov == bv && ox < bx);
+                    bv = take ? ov : bv;
+                    bx = take ? ox : bx;
+                }
+                if (v[0] != -INFINITY && ix[0] == bx) {
+                    v[0] = v[1];
+                    v[1] = v[2];
+                    v[2] = v[3];
+                    v[3] = -INFINITY;
+                    ix[0] = ix[1];
+                    ix[1] = ix[2];
+                    ix[2] = ix[3];
+                }
+                if (lane == t) {
+                    kv[k] = bv;
+                    kx[k] = bx == 0xFFFFFFFFu ? 0u : bx;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                v[k] = kv[k];
+                ix[k] = kx[k];
+            }
+        }
+        if (ok) {
+            uint32_t cb[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const bool filled = v[k] != -INFINITY;
+                cb[k] = filled ? (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v[k]) : 0u;
+                ix[k] = filled ? ix[k] : 0u;
+            }
+            const uint4_t code = {ix[0] | (ix[1] << 16), ix[2] | (ix[3] << 16), cb[0] | (cb[1] << 16), cb[2] | (cb[3] << 16)};
+            a.cold[(uint64_t)c * kBlockTokens * a.kv_heads + tt3 * a.s_tok + g * a.s_head] = code;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); // the list is read before the next tile's is written
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
+
+// Variance proxy of each listed block (distiller.rs:126-159), bit-exact: the
+// reference's loops in memory order, in f64, with no fused multiply-add (the
+// reference squares, then adds), and returns f32; an all-zero block gives 0.
+// Without a block list (src null) entry i takes block i.
+//
+// The f64 sum of the squares is one sequential chain of adds per block; everything
+// before the add is not.  A work-group owns kEntBlocks blocks: four waves, 16 threads
+// per block, load the values (kEntAhead chunks ahead) and write each value's term to
+// LDS, and the lanes of a fifth wave, one per block, only add, a chunk behind.  A
+// chunk's tile is written while the other one is added, one barrier a chunk.
+// Bound: the chain of dependent adds (7 ns each; 115 of 165 us for one work-group of
+// 16384-value blocks) and, with two work-groups per CU, the first pass's loads: 8192
+// such blocks 404 -> 214 us, 16 404 -> 166, against one wave per 16 blocks whose chain
+// lanes converted, subtracted and squared as well.
+constexpr int kEntChunk = 128;                // values per block and chunk (256 bytes)
+constexpr int kEntCols = kEntChunk / 8;       // 16-byte words per block and chunk, one per thread
+constexpr int kEntAhead = 4;
+constexpr int kEntPitch = kEntChunk + 2;      // row of terms, in doubles: 16 rows read one column without conflicts
+constexpr int kEntBlocks = 16;
+constexpr int kEntThreads = kEntBlocks * kEntCols + 64;
 
 // The sum of a block's values needs no particular order when it is exact:
 // f16 values are multiples of 2^-24, so when sum|v| < 2^29 every partial sum of
 // any subset is a multiple of 2^-24 below 2^53 of them, exactly representable
 // in f64, and the reference's sequential sum from -0.0 equals any other order
 // (a zero total is +0.0 both ways unless every value is a zero, and then the
-// proxy is 0 anyway).  Pass 0 sums in four independent chains and records
-// sum|v| and whether an inf or NaN occurred; a wave with a block outside the
-// exact case repeats the sum sequentially (pass 2).
+// proxy is 0 anyway).  The first pass sums in four independent chains a thread
+// and records sum|v| and whether an inf or NaN occurred; a work-group with a block
+// outside the exact case repeats the sum sequentially.
 constexpr int kEntChains = 4;
 struct EntSum {
     double s[kEntChains], m[kEntChains];
     bool all_zero, nonfinite;
 };
 
-// One 16-byte word (8 values) of a block, in memory order: pass 0 adds the
-// values in kEntChains chains (and their magnitudes), pass 1 adds the squared
-// deviations, pass 2 adds the values sequentially.
-template <int PASS>
-__device__ inline void entropy_word(const uint4_t w, EntSum& st, double& acc, double mean) {
+// The 8 values of a 16-byte word into the order-free sums of pass 0.
+__device__ inline void entropy_add(const uint4_t w, EntSum& st) {
 #pragma clang fp contract(off)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const uint32_t bits = (w[e / 2] >> (16 * (e % 2))) & 0xFFFFu;
         const float f = h2f_bits(bits);
-        if constexpr (PASS == 0) {
-            st.all_zero = st.all_zero && f == 0.0f;
-            st.nonfinite = st.nonfinite || ((bits >> 10) & 31u) == 31u;
-            st.s[e % kEntChains] = st.s[e % kEntChains] + (double)f;
-            st.m[e % kEntChains] = st.m[e % kEntChains] + (double)fabsf(f);
-        } else if constexpr (PASS == 1) {
-            const double diff = (double)f - mean;
-            const double sq = diff * diff;
-            acc = acc + sq;
-        } else {
-            acc = acc + (double)f;
-        }
+        st.all_zero = st.all_zero && f == 0.0f;
+        st.nonfinite = st.nonfinite || ((bits >> 10) & 31u) == 31u;
+        st.s[e % kEntChains] = st.s[e % kEntChains] + (double)f;
+        st.m[e % kEntChains] = st.m[e % kEntChains] + (double)fabsf(f);
     }
 }
 
-// Blocks per wave.  A wave's 64 lanes all load (the stream is latency-bound:
-// more waves keep more chunks in flight) and all sum the values for the mean,
-// four lanes per block; the first kEntBlocks lanes run the sequential chains
-// (the variance, and the mean when its sums are not exact).  At 16 blocks a
-// wave, 8192 blocks make 512 waves.
-constexpr int kEntBlocks = 16;
-
-__global__ __launch_bounds__(64) void entropy_kernel(EncodeArgs a, uint32_t head_dim) {
-    constexpr int NB = kEntBlocks, PL = NB * kEntCols / 64; // 16-byte loads per lane and chunk
-    static_assert(PL * 64 == NB * kEntCols, "chunk loads");
-    static_assert(NB * 4 == 64 && kEntCols % 4 == 0, "four lanes per block in the mean pass");
-    __shared__ uint4_t tile[2][NB][kEntPitch];
-    __shared__ uint32_t s_blk[NB];
-    const uint32_t lane = threadIdx.x;
-    const bool chain = lane < (uint32_t)NB; // this lane owns a block
-    const uint32_t i = blockIdx.x * NB + lane;
+__global__ __launch_bounds__(kEntThreads) __attribute__((amdgpu_waves_per_eu(3))) void entropy_kernel(EncodeArgs a, uint32_t head_dim) {
+#pragma clang fp contract(off)
+    constexpr int NB = kEntBlocks, COLS = kEntCols;
+    __shared__ __attribute__((aligned(16))) double tile[2][NB][kEntPitch];
+    __shared__ double s_mean[NB];
+    __shared__ uint32_t s_flags[NB]; // 1: all zero, 2: the sum depends on its order
+    const uint32_t tid = threadIdx.x, r = tid / COLS, c = tid % COLS;
+    const bool adder = tid >= (uint32_t)(NB * COLS);
+    const uint32_t row = adder ? tid - NB * COLS : r; // the adders' lanes past NB idle
+    const uint32_t i = blockIdx.x * NB + row;
     uint32_t b = 0;
     bool ok = false;
-    if (chain && i < a.n_blocks) {
+    if (row < (uint32_t)NB && i < a.n_blocks) {
         b = a.src ? (a.src[i] & kRefMask) : i;
         ok = b < a.hot_blocks;
-        if (!ok) flag_error(a.err, kErrHotRef);
+        if (!ok && adder) flag_error(a.err, kErrHotRef);
     }
-    if (chain) s_blk[lane] = ok ? b : 0xFFFFFFFFu;
-    __syncthreads();
     const uint64_t n = (uint64_t)kBlockTokens * a.kv_heads * head_dim; // values per block
     const uint64_t words = n / 8;                                        // 16-byte words per block
-    const uint64_t n_chunks = (words + kEntCols - 1) / kEntCols;
-    const uint4_t* hot = (const uint4_t*)a.hot;
-    // Lane l loads words (k * 64 + l) of the chunk: row r = that / kEntCols, column c.
-    uint4_t reg[PL];
-    auto load = [&](uint64_t ch) {
+    const uint64_t n_chunks = (words + COLS - 1) / COLS;
+    const uint4_t* hot = (const uint4_t*)a.hot + (uint64_t)(ok ? b : 0u) * words;
+    if (!adder) {
+        EntSum st;
 #pragma unroll
-        for (int k = 0; k < PL; ++k) {
-            const uint32_t idx = k * 64 + lane, r = idx / kEntCols, c = idx % kEntCols;
-            const uint32_t rb = s_blk[r];
-            const uint64_t w = ch * kEntCols + c;
-            reg[k] = (rb != 0xFFFFFFFFu && w < words) ? hot[(uint64_t)rb * words + w] : uint4_t{0, 0, 0, 0};
-        }
-    };
-    auto store = [&](int buf) {
+        for (int k = 0; k < kEntChains; ++k) st.s[k] = st.m[k] = -0.0;
+        st.all_zero = true;
+        st.nonfinite = false;
+        if (ok) {
+            constexpr int U = 8; // loads in flight
+            uint64_t w = c;
+            for (; w + (U - 1) * COLS < words; w += U * COLS) {
+                uint4_t v[U];
 #pragma unroll
-        for (int k = 0; k < PL; ++k) {
-            const uint32_t idx = k * 64 + lane;
-            tile[buf][idx / kEntCols][idx % kEntCols] = reg[k];
-        }
-    };
-    EntSum st;
+                for (int u = 0; u < U; ++u) v[u] = hot[w + u * COLS];
 #pragma unroll
-    for (int k = 0; k < kEntChains; ++k) st.s[k] = st.m[k] = -0.0;
-    st.all_zero = true;
-    st.nonfinite = false;
-    double mean = 0.0;
-    // Streams the whole block once per pass; the pass is a compile-time constant
-    // so the inner loops carry no branch.
-    auto stream = [&](auto pass, double acc) {
-        constexpr int P = decltype(pass)::value;
-        load(0);
-        store(0);
-        __syncthreads();
-        for (uint64_t ch = 0; ch < n_chunks; ++ch) {
-            const int cur = (int)(ch & 1);
-            const bool more = ch + 1 < n_chunks;
-            if (more) load(ch + 1);
-            if constexpr (P == 0) {
-                // Every lane: a quarter of the words of block lane / 4 (exact sums
-                // are the same in any order; the quarters are added after the pass).
-                constexpr uint32_t QW = kEntCols / 4;
-                const uint4_t* row = tile[cur][lane / 4];
-                const uint32_t cols = (ch + 1) * kEntCols <= words ? (uint32_t)kEntCols : (uint32_t)(words - ch * kEntCols);
-                const uint32_t c0 = (lane % 4) * QW;
-#pragma unroll
-                for (uint32_t c = 0; c < QW; ++c)
-                    if (c0 + c < cols) entropy_word<0>(row[c0 + c], st, acc, mean);
-            } else if (chain) {
-                const uint4_t* row = tile[cur][lane];
-                if ((ch + 1) * kEntCols <= words) {
-                    uint4_t w[kEntCols];
-#pragma unroll
-                    for (int c = 0; c < kEntCols; ++c) w[c] = row[c];
-#pragma unroll
-                    for (int c = 0; c < kEntCols; ++c) entropy_word<P>(w[c], st, acc, mean);
-                } else {
-                    const uint32_t cols = (uint32_t)(words - ch * kEntCols);
-                    for (uint32_t c = 0; c < cols; ++c) entropy_word<P>(row[c], st, acc, mean);
-                }
+                for (int u = 0; u < U; ++u) entropy_add(v[u], st);
             }
-            if (more) store(cur ^ 1);
-            __syncthreads();
+            for (; w < words; w += COLS) entropy_add(hot[w], st);
         }
+        // The 16 threads' sums (exact whenever the test below passes).
+        double sum = (st.s[0] + st.s[1]) + (st.s[2] + st.s[3]), mag = (st.m[0] + st.m[1]) + (st.m[2] + st.m[3]);
+        uint32_t az = st.all_zero ? 1u : 0u, nf = st.nonfinite ? 1u : 0u;
+#pragma unroll
+        for (int o = 1; o < COLS; o *= 2) {
+            sum += __shfl_xor(sum, o);
+            mag += __shfl_xor(mag, o);
+            az &= (uint32_t)__shfl_xor((int)az, o);
+            nf |= (uint32_t)__shfl_xor((int)nf, o);
+        }
+        if (c == 0) {
+            s_mean[r] = sum / (double)n;
+            s_flags[r] = az | (nf || !(mag < 536870912.0) ? 2u : 0u); // 2^29
+        }
+    }
+    __syncthreads();
+    // The sequential sum over the block of the values (SQ false) or of their squared
+    // deviations from the mean, in the adders' lanes.  Terms past the block's end are
+    // -0.0, which leaves any sum as it is.
+    auto chain = [&](auto squares) {
+        constexpr bool SQ = decltype(squares)::value;
+        const double mean = row < (uint32_t)NB ? s_mean[row] : 0.0;
+        double acc = -0.0;
+        auto load = [&](uint64_t ch) {
+            const uint64_t w = ch * COLS + c;
+            return ok && w < words ? hot[w] : (uint4_t)0u;
+        };
+        auto put = [&](uint64_t ch, const uint4_t v) {
+            double t[8];
+            const bool in = ch * COLS + c < words;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const double f = (double)h2f_bits((v[e / 2] >> (16 * (e % 2))) & 0xFFFFu);
+                const double d = f - mean;
+                t[e] = in ? (SQ ? d * d : f) : -0.0;
+            }
+            double* to = &tile[ch & 1u][r][8 * c];
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) *(double2_t*)(to + e) = (double2_t){t[e], t[e + 1]};
+        };
+        auto add = [&](uint64_t ch) {
+            const double2_t* from = (const double2_t*)tile[ch & 1u][row];
+            constexpr int G = 8; // pairs read ahead of the adds
+            double2_t cur[G], nxt[G];
+#pragma unroll
+            for (int k = 0; k < G; ++k) cur[k] = from[k];
+#pragma unroll 1
+            for (int q = 0; q < kEntChunk / 2; q += G) {
+                const int ahead = q + G < kEntChunk / 2 ? q + G : q;
+#pragma unroll
+                for (int k = 0; k < G; ++k) nxt[k] = from[ahead + k];
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    acc = acc + cur[k][0];
+                    acc = acc + cur[k][1];
+                }
+#pragma unroll
+                for (int k = 0; k < G; ++k) cur[k] = nxt[k];
+            }
+        };
+        uint4_t v[kEntAhead];
+        if (!adder)
+#pragma unroll
+            for (int k = 0; k < kEntAhead; ++k) v[k] = load((uint64_t)k);
+        for (uint64_t ch0 = 0; ch0 < n_chunks; ch0 += kEntAhead) {
+#pragma unroll
+            for (int k = 0; k < kEntAhead; ++k) {
+                const uint64_t ch = ch0 + (uint64_t)k;
+                if (ch >= n_chunks) break; // uniform
+                if (!adder) {
+                    put(ch, v[k]);
+                    v[k] = load(ch + kEntAhead);
+                }
+                __syncthreads(); // tile ch is whole; tile ch - 1 has been added
+                if (adder && row < (uint32_t)NB) add(ch);
+            }
+        }
+        __syncthreads();
         return acc;
     };
-    (void)stream(std::integral_constant<int, 0>{}, -0.0);
-    // Lanes 4r .. 4r+3 hold block r's quarter sums: added (exact whenever the
-    // test below passes) and handed to lane r, the block's owner.
-    double s4 = (st.s[0] + st.s[1]) + (st.s[2] + st.s[3]);
-    double m4 = (st.m[0] + st.m[1]) + (st.m[2] + st.m[3]);
-    uint32_t az = st.all_zero ? 1u : 0u, nf = st.nonfinite ? 1u : 0u;
-#pragma unroll
-    for (int o = 1; o < 4; o *= 2) {
-        s4 += __shfl_xor(s4, o);
-        m4 += __shfl_xor(m4, o);
-        az &= (uint32_t)__shfl_xor((int)az, o);
-        nf |= (uint32_t)__shfl_xor((int)nf, o);
+    const bool ordered = row < (uint32_t)NB && (s_flags[row] & 2u);
+    if (__syncthreads_or(ordered ? 1 : 0)) { // some block's sum depends on its order
+        const double seq = chain(std::false_type{});
+        if (adder && ordered) s_mean[row] = seq / (double)n;
+        __syncthreads();
     }
-    const int src = (int)(chain ? lane * 4u : 0u);
-    double sum = __shfl(s4, src);
-    const double mag = __shfl(m4, src);
-    st.all_zero = __shfl((int)az, src) != 0;
-    st.nonfinite = __shfl((int)nf, src) != 0;
-    const bool exact = !chain || (!st.nonfinite && mag < 536870912.0); // 2^29
-    if (__any(!exact)) { // wave-uniform: the sequential sum for the blocks that need it
-        const double seq = stream(std::integral_constant<int, 2>{}, -0.0);
-        sum = exact ? sum : seq;
-    }
-    mean = sum / (double)n;
-    const double var = stream(std::integral_constant<int, 1>{}, -0.0);
-    if (chain && i < a.n_blocks) a.entropy[i] = (!ok || st.all_zero) ? 0.0f : (float)(var / (double)n);
+    const double var = chain(std::true_type{});
+    if (adder && row < (uint32_t)NB && i < a.n_blocks)
+        a.entropy[i] = (!ok || (s_flags[row] & 1u)) ? 0.0f : (float)(var / (double)n);
 }
 
 } // namespace aw

@@ -201,3 +201,43 @@ def test_encode_prefilter_matches_full_scan(engine, stream, case):
     want = oracle.encode_blocks(hb, db, src, cold=cold0.copy())
     assert (scan == want).all()
     assert (got == want).all(), f"{int((got != want).any(axis=-1).sum())} codes differ"
+
+
+# (kv_heads, head_dim, atoms, dict_heads, blocks): dictionaries that just fit in LDS and just do not
+# (128 KiB a head), the smallest, an odd number of 16-atom tiles, one dictionary for all heads, one
+# block, and more 64-token tiles than a work-group has waves.
+RESIDENT = [(4, 128, 512, 4, 5), (4, 128, 528, 4, 5), (2, 64, 1024, 2, 9), (2, 64, 1040, 1, 3), (3, 64, 16, 1, 1),
+            (1, 128, 48, 1, 70), (8, 128, 496, 1, 33)]
+
+
+@pytest.mark.parametrize("hkv,hd,a,dheads,nb", RESIDENT, ids=["-".join(map(str, c)) for c in RESIDENT])
+def test_encode_resident_dictionary_edges(engine, stream, hkv, hd, a, dheads, nb):
+    """The prefilter with the dictionary in LDS (and, past its size, the streamed one)
+    against the exact scan, bit for bit: zero and one-hot tokens (all scores tied),
+    tokens whose scores are all negative, products near the largest and the
+    smallest, an atom of a far larger norm, inf and NaN atoms and tokens."""
+    rng = np.random.default_rng(a * 7 + nb)
+    hot = rng.standard_normal((nb, 16, hkv, hd)).astype(np.float16)
+    d = _unit(rng, (dheads, a, hd))
+    d[:, 5] *= np.float16(300)
+    d[:, a - 1] = -d[:, 5]
+    hot[0, 0] = 0
+    hot[0, 1] = 0
+    hot[0, 1, :, 3] = 1
+    hot[0, 2] *= np.float16(2.0 ** -14)
+    hot[0, 3] = np.float16(2.0 ** -24)
+    hot[0, 4] = np.copysign(np.float16(60000), hot[0, 4])
+    hot[0, 5, 0, 1] = np.nan
+    hot[0, 6, hkv - 1, 2] = -np.inf
+    d[0, 8:14] = -np.abs(d[0, 8:14])
+    hot[0, 7] = np.abs(hot[0, 7])
+    if nb % 2:
+        d[dheads - 1, 7, 0] = np.inf
+        d[dheads - 1, a - 2, hd - 1] = np.nan
+    hb, db, src = hot.view(np.uint16), d.view(np.uint16), rng.permutation(nb)
+    cold0 = np.zeros((nb, 16, hkv, 8), np.uint16)
+    got, _ = run_device(engine, stream, hb, db, src, None, cold0.copy(), False, False)
+    want = oracle.encode_blocks(hb, db, src, cold=cold0.copy())
+    assert (got == want).all(), f"{int((got != want).any(axis=-1).sum())} codes differ"
+    scan, _ = run_device(engine, stream, hb, db, src, None, cold0.copy(), False, False, full_scan=True)
+    assert (scan == want).all()
