@@ -287,10 +287,13 @@ int aw_ops_rope(aw_engine* e, uint16_t* q, uint16_t* k, uint32_t num_tokens, uin
     if (head_dim == 0 || head_dim % 2) return ei::fail(e, AW_E_INVALID_ARG, "rope: head_dim %u must be even", head_dim);
     if ((q_heads && !q) || (kv_heads && !k)) return ei::fail(e, AW_E_INVALID_ARG, "rope: null pointer");
     if (!(theta > 0.0f)) return ei::fail(e, AW_E_INVALID_ARG, "rope: theta must be positive");
-    const uint64_t threads = (uint64_t)num_tokens * ((uint64_t)q_heads + kv_heads) * (head_dim / 2);
-    if (cdiv64(threads, 256) > 0x7FFFFFFFull) return ei::fail(e, AW_E_UNSUPPORTED, "rope: grid too large");
-    hipLaunchKernelGGL(awo::rope_kernel, dim3((uint32_t)cdiv64(threads, 256)), dim3(256), 0, (hipStream_t)stream, q, k,
-                       num_tokens, q_heads, kv_heads, head_dim, start_position, theta);
+    const uint64_t heads = (uint64_t)q_heads + kv_heads, pairs = (uint64_t)num_tokens * (head_dim / 2);
+    if (cdiv64(pairs * heads, 256) > 0x7FFFFFFFull) return ei::fail(e, AW_E_UNSUPPORTED, "rope: grid too large");
+    // Heads of one thread: as many as leave every CU two work-groups, at most 8 (a
+    // longer run is a longer chain of loads).
+    const uint32_t per = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(8, pairs * heads / (512ull * ei::compute_units(e))));
+    hipLaunchKernelGGL(awo::rope_kernel, dim3((uint32_t)cdiv64(pairs * cdiv64(heads, per), 256)), dim3(256), 0,
+                       (hipStream_t)stream, q, k, num_tokens, q_heads, kv_heads, head_dim, start_position, theta, per);
     OPS_HIP(e, hipGetLastError());
     return AW_OK;
 }

@@ -192,23 +192,31 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* in, const
 // (x[p], x[p + hd/2]) of each head rotates by angle = f32(start + t) * freq_p,
 // freq_p = 1 / theta^(2p/hd).  freq_p is the double-precision value rounded
 // to fp32; cos and sin of the fp32 angle are taken in double and rounded to
-// fp32; the rotation itself is fp32, one rounding per operation.  Thread =
-// (pair, head row, token); head rows 0 .. Hq-1 are q, Hq .. Hq+Hkv-1 are k.
+// fp32; the rotation itself is fp32, one rounding per operation.
+//
+// Thread = (pair, token, group of heads): the double-precision power, cosine and sine
+// (the bound when each pair of each head took its own) once for `per` heads of the
+// token; heads 0 .. Hq-1 are q, Hq .. Hq+Hkv-1 are k.  512 tokens of 32 + 8 heads x
+// 128 dims: 18.3 -> 8.0 us.
 __global__ __launch_bounds__(256) void rope_kernel(uint16_t* q, uint16_t* k, uint32_t T, uint32_t Hq, uint32_t Hkv,
-                                                   uint32_t hd, uint32_t start, float theta) {
-    const uint32_t half_dim = hd / 2;
+                                                   uint32_t hd, uint32_t start, float theta, uint32_t per) {
+    const uint32_t half_dim = hd / 2, heads = Hq + Hkv;
+    const uint32_t groups = (heads + per - 1) / per;
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t per_tok = (uint64_t)(Hq + Hkv) * half_dim;
-    if (i >= per_tok * T) return;
-    const uint32_t t = (uint32_t)(i / per_tok), rem = (uint32_t)(i % per_tok);
-    const uint32_t head = rem / half_dim, pr = rem % half_dim;
+    if (i >= (uint64_t)T * groups * half_dim) return;
+    const uint32_t pr = (uint32_t)(i % half_dim);
+    const uint64_t tg = i / half_dim;
+    const uint32_t h0 = (uint32_t)(tg % groups) * per, h1 = min(h0 + per, heads);
+    const uint64_t t = tg / groups;
     const float freq = (float)(1.0 / pow((double)theta, (double)(2 * pr) / (double)hd));
-    const float angle = (float)(start + t) * freq;
+    const float angle = (float)(start + (uint32_t)t) * freq;
     const float c = (float)cos((double)angle), s = (float)sin((double)angle);
-    uint16_t* base = head < Hq ? q + ((uint64_t)t * Hq + head) * hd : k + ((uint64_t)t * Hkv + (head - Hq)) * hd;
-    const float x0 = h2f(base[pr]), x1 = h2f(base[pr + half_dim]);
-    base[pr] = f2h(x0 * c - x1 * s);
-    base[pr + half_dim] = f2h(x0 * s + x1 * c);
+    for (uint32_t head = h0; head < h1; ++head) {
+        uint16_t* base = head < Hq ? q + (t * Hq + head) * hd : k + (t * Hkv + (head - Hq)) * hd;
+        const float x0 = h2f(base[pr]), x1 = h2f(base[pr + half_dim]);
+        base[pr] = f2h(x0 * c - x1 * s);
+        base[pr + half_dim] = f2h(x0 * s + x1 * c);
+    }
 }
 
 // ------------------------------------------------------- C = A . B^T
