@@ -423,8 +423,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(GemmArgs a) {
     }
 }
 
-// Products of more than 64 rows whose rows are not 16-byte aligned (or are of
-// 2 MiB): 128 x 128 output tiles, 4 waves of 64 x 64 (4 x 4 MFMA tiles each), k-steps
+// Products of more than 64 rows whose rows are not 16-byte aligned (or are over
+// 4 MiB): 128 x 128 output tiles, 4 waves of 64 x 64 (4 x 4 MFMA tiles each), k-steps
 // of 32 staged in LDS with the next step's loads in registers while the current step
 // is multiplied.  One weight matrix (group 0).  The steps are summed in the order of
 // gemm_tile_kernel, so both give the same bits.  Bound: the gathered loads.
