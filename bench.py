@@ -554,9 +554,9 @@ def encoder_bench(engine, seed, reps, cpu_blocks):
             "token_heads_per_s": round(tok_heads / (ms * 1e-3), 1),
             "achieved_tflops": round(tf, 2),
             "roofline": {"bound": "mfma", "peak_tflops": MFMA_F16_TFLOPS, "frac": round(tf / MFMA_F16_TFLOPS, 4),
-                         "note": "the projection x . D^T (counted once) runs twice on MFMA, f16 in, f32 out, then the "
-                                 "candidate atoms are rescored in the reference's fp32 order; the per-score bound and "
-                                 "top-4 bookkeeping on the VALU bounds the kernel, not the matrix cores"},
+                         "note": "the projection x . D^T runs on MFMA, f16 in, f32 out, then the candidate atoms are "
+                                 "rescored in the reference's fp32 order; keeping each lane's five best scores on "
+                                 "the VALU bounds the kernel, not the matrix cores"},
             "full_scan": {"ms_per_call": round(scan_ms, 4), "achieved_tflops": round(scan_tf, 2),
                           "valu_frac": round(scan_tf / VALU_FP32_FMA_TFLOPS, 4), "valu_peak_tflops": VALU_FP32_FMA_TFLOPS,
                           "note": "AW_F_ENCODE_FULL_SCAN: one exact fp32 FMA per (token, kv head, atom, dim); same codes"},
