@@ -40,22 +40,23 @@ struct PrefillArgs {
 // Staged rows are HD / 8 16-byte chunks, chunk c of K row r at c ^ (r % chunks),
 // of V row r at c ^ 4 (r % 4) ^ (r / 4) % 4 (128 dims) so that the 4 rows of a
 // transposing read lie in different quarters: no bank conflict at 128 dims.
-// A row's sums are rescaled only when its maximum grew by more than 2^8; the
-// weights in 16 bits then no longer hold each group's largest exactly, as the
-// decode kernel's do, so half of them (the first 32 positions of a step) are
-// multiplied as two f16 terms: error against 64 bits 2.3e-4 of the result at
-// 2048 positions (2.6e-4 without, 2.4e-4 in groups of decodes).
-// Bound: a wave's own chain of products, softmax, products (1.5 us a step with one
-// wave per SIMD, 1.3 a wave with two; MFMA busy 49% of the cycles).
-// 2048 queries of 32 heads x 128 dims: 2930 -> 60 us (0.57 PFLOP/s of the pairs
+// A row's sums are rescaled whenever its maximum grows: its largest weight so far is
+// exactly 1, as in the decode kernel, whose 32-position groups the second half of a
+// step equals.  The first 32 positions' weights, whose maximum the second half may
+// still raise, are multiplied as two f16 terms.  Error against 64 bits, against groups
+// of decodes: random scores 2.1e-4 (2.4e-4) at 600 positions, 2.4e-4 (2.6e-4) at 2000;
+// rows where a later position takes most of the weight equal to within 0.2%.  (Rescaled
+// only after a growth of 2^8: 62.8 us instead of 66.4 at 2048 queries, and such rows
+// up to 27% above; without the second term 59.4 us and up to 7% above; with it for
+// all positions 69.2.)
+// Bound: a wave's own chain of products, softmax, products.
+// 2048 queries of 32 heads x 128 dims: 2930 -> 66 us (0.52 PFLOP/s of the pairs
 // that are seen), against 128 decodes of 16 queries each; 509 of 14 x 64 behind
-// 1022 positions 585 -> 20 us.
+// 1022 positions 585 -> 19 us.
 constexpr int kPrefillRows = 128;   // query rows of one kv head per work-group: 4 waves x 32
 constexpr int kPrefillTokens = 64;  // cache tokens per staged tile
 constexpr int kPrefillThreads = 256;
 constexpr size_t prefill_lds_bytes(int HD) { return (size_t)2 * 2 * kPrefillTokens * HD * 2; }
-// log2 a row's maximum may grow before its sums are rescaled: p <= 2^8 stays far inside f16.
-constexpr float kPrefillLazy = 8.0f;
 
 // One row of one split by one wave, without matrix instructions: positions
 // [c0, min(c1, the row's limit)).
@@ -229,7 +230,7 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
         const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, mx), __builtin_bit_cast(uint32_t, mx), false, false);
         const uint32_t sw0 = sw[0], sw1 = sw[1]; // the row's two halves
         mx = fmaxf(__builtin_bit_cast(float, sw0), __builtin_bit_cast(float, sw1)) * a.scale_log2;
-        if (__any(mx > m_run + kPrefillLazy)) {
+        if (__any(mx > m_run)) {
             const float mnew = fmaxf(m_run, mx);
             const float alpha = mnew == -INFINITY ? 1.0f : fast_exp2(m_run - mnew);
             m_run = mnew;

@@ -497,3 +497,44 @@ def test_prompt_attention_captured_without_workspace(stream):
         eng.multihead_attention(qt, kt, vt, eager, kv_len, d, hq, hkv, nq, cache_tokens=kv_len)
         assert_close(eager.double().cpu().numpy(), ref)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("nq,kv_len,hq,hkv,d", [
+    (600, 600, 8, 2, 128),  # one part
+    (320, 320, 4, 4, 64),
+    (300, 1100, 32, 8, 128),  # several parts of several steps
+    (300, 1100, 14, 2, 64),
+])
+@pytest.mark.parametrize("growth", [3.0, 7.75])
+def test_prompt_attention_peaked_rows(engine, stream, nq, kv_len, hq, hkv, d, growth):
+    """Rows whose maximum grows in a later step, by a position that then takes most of
+    the weight: every 64th position has 2^0, one position in each half of a step
+    2^growth, the others 2^-14.  The error against 64 bits is no larger than that
+    of the few-query kernel on the same rows (its rounding of the weights is the
+    reference: a row's largest is exactly 1); 5% for the two orders of sums, whose
+    effect on the root mean square over 40 thousand values or more is below 1%."""
+    cap = -(-kv_len // 16) * 16
+    q, k, v = cache_case(int(growth) + nq + d, nq, kv_len, hq, hkv, d, cap)
+    scores = np.full(cap, -14.0)
+    scores[::64] = 0.0
+    first = kv_len - nq
+    for i, at in enumerate((64 + 45, 64 * (kv_len // 64 - 1) + 10)):
+        scores[at] = growth - 0.25 * i
+    k[..., 1:] *= np.float16(0.01)
+    q[..., 0] = np.float16(8.0)
+    k[..., 0] = (scores * np.sqrt(d) / (8.0 * np.log2(np.e)))[:, None]
+    qt, kt, vt = (torch.from_numpy(x.view(np.int16)).cuda() for x in (q, k, v))
+    out = torch.empty((nq, hq, d), dtype=torch.float16, device="cuda:0")
+    few = torch.empty_like(out)
+    engine.multihead_attention(qt, kt, vt, out, kv_len, d, hq, hkv, nq, cache_tokens=cap, stream=stream)
+    for i in range(0, nq, 9):  # 9 queries of 7 heads are one decode still
+        n = min(9, nq - i)
+        engine.multihead_attention(qt[i:i + n], kt, vt, few[i:i + n], first + i + n, d, hq, hkv, n, cache_tokens=cap,
+                                   stream=stream)
+    engine.check_device_errors(stream)
+    ref = AO.multihead_attention_f64(q, k[:kv_len], v[:kv_len], kv_len, nq)
+    rel = [float(np.linalg.norm(t.double().cpu().numpy() - ref) / np.linalg.norm(ref)) for t in (out, few)]
+    print(f"peaked rows: nq {nq} kv_len {kv_len} d {d} growth {growth}: rel-L2 {rel[0]:.3e}, few-query {rel[1]:.3e}",
+          flush=True)
+    assert_close(out.double().cpu().numpy(), ref)
+    assert rel[0] <= 1.05 * rel[1], rel
