@@ -58,55 +58,15 @@ constexpr int kPrefillTokens = 64;  // cache tokens per staged tile
 constexpr int kPrefillThreads = 256;
 constexpr size_t prefill_lds_bytes(int HD) { return (size_t)2 * 2 * kPrefillTokens * HD * 2; }
 
-// One row of one split by one wave, without matrix instructions: positions
-// [c0, min(c1, the row's limit)).
-template <int HD>
-__device__ __forceinline__ void prefill_row(const PrefillArgs& a, uint32_t g, uint32_t s, uint32_t r, uint32_t c0,
-                                                      uint32_t c1) {
-    constexpr int DL = HD / 64; // dims per lane
-    const uint32_t lane = threadIdx.x & 63u, qi = r / a.gqa;
-    const uint64_t row = (uint64_t)qi * a.q_heads + g * a.gqa + r % a.gqa;
-    const uint32_t end = min(c1, a.kv_len - a.n + 1u + qi);
-    float q[DL], o[DL], m = -INFINITY, l = 0.0f;
+// x with its infinities and NaNs replaced by zeros.
+__device__ __forceinline__ half8_t finite_part(half8_t x) {
+    uint4_t w = __builtin_bit_cast(uint4_t, x);
 #pragma unroll
-    for (int d = 0; d < DL; ++d) {
-        q[d] = h2f_bits(a.q[row * HD + d * 64 + lane]);
-        o[d] = 0.0f;
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t v = w[e];
+        w[e] = ((v & 0x7C00u) == 0x7C00u ? 0u : v & 0xFFFFu) | ((v & 0x7C000000u) == 0x7C000000u ? 0u : v & 0xFFFF0000u);
     }
-    constexpr int U = 4; // positions whose loads and sums overlap
-    for (uint32_t c = c0; c < end; c += U) {
-        float x[U], v[U][DL];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint64_t at = ((uint64_t)min(c + u, end - 1u) * a.kv_heads + g) * HD + lane;
-            x[u] = 0.0f;
-#pragma unroll
-            for (int d = 0; d < DL; ++d) {
-                x[u] = fmaf(q[d], h2f_bits(a.k[at + d * 64]), x[u]);
-                v[u][d] = h2f_bits(a.v[at + d * 64]);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const float y = wave_sum(x[u]) * a.scale_log2;
-            if (c + u >= end || y == -INFINITY) continue;
-            const float mnew = fmaxf(m, y), alpha = fast_exp2(m - mnew), p = fast_exp2(y - mnew);
-            l = l * alpha + p;
-#pragma unroll
-            for (int d = 0; d < DL; ++d) o[d] = fmaf(p, v[u][d], o[d] * alpha);
-            m = mnew;
-        }
-    }
-    const uint64_t at = ((uint64_t)g * a.splits + s) * a.rows + r;
-    if (a.splits > 1u && lane == 0) {
-        a.part_m[at] = m;
-        a.part_l[at] = l;
-    }
-#pragma unroll
-    for (int d = 0; d < DL; ++d) {
-        if (a.splits > 1u) a.part_o[at * HD + d * 64 + lane] = o[d];
-        else a.out[row * HD + d * 64 + lane] = __builtin_bit_cast(uint16_t, (_Float16)(l == 0.0f ? 0.0f : o[d] / l));
-    }
+    return as_h8(w);
 }
 
 template <int HD>
@@ -180,10 +140,8 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
         __asm__ volatile("" ::: "memory");
     };
 
-    float m_run = -INFINITY, l_run = 0.0f;
+    float m_run, l_run;
     float16_t oacc[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) oacc[nb] = (float16_t)0.0f;
 
     // LDS offsets (halves) of this lane's operands in a staged tile.
     uint32_t kat[KS], va[NB], vb[NB];
@@ -199,7 +157,10 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
         }
     }
 
-    auto process = [&](uint32_t tt, uint32_t buf) {
+    // SPLIT: the products take the values' finite part, and positions with an inf or NaN
+    // are then added to the rows that see them one by one, weights in f32.
+    auto process = [&](auto split, uint32_t tt, uint32_t buf) {
+        constexpr bool SPLIT = decltype(split)::value;
         const int c0 = (int)(tt * (uint32_t)kPrefillTokens);
         if (c0 >= wmax) return; // wave-uniform: every row of the wave ends before this tile
         const _Float16* sb = pre_lds + buf * 2u * OP;
@@ -266,46 +227,105 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
         for (int x = 0; x < 4 * NB; ++x) {
             const int tb = x / (2 * NB), kk = (x / NB) % 2, nb = x % NB;
-            const half8_t v = vfrag(tb, kk, nb);
+            half8_t v = vfrag(tb, kk, nb);
+            if constexpr (SPLIT) v = finite_part(v);
             oacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, pop[tb][kk], oacc[nb], 0, 0, 0);
             if (tb == 0) oacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, plo[kk], oacc[nb], 0, 0, 0);
+            if constexpr (SPLIT) __builtin_amdgcn_sched_barrier(0); // fewer fragments at once: no spills
+        }
+        if constexpr (SPLIT) {
+            // Whether slot c of the tile's row holds an inf or NaN.
+            auto nonfinite = [&](uint32_t row, uint32_t c) -> bool {
+                const uint4_t w = *(const uint4_t*)(sb + OP + row * HD + 8u * c);
+                bool any = false;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t v = w[e];
+                    any |= (v & 0x7C00u) == 0x7C00u || (v & 0x7C000000u) == 0x7C000000u;
+                }
+                return any;
+            };
+            bool any = false; // row `lane`, from another slot on in each lane (banks)
+#pragma unroll 4
+            for (uint32_t c = 0; c < (uint32_t)CH; ++c) any |= nonfinite((uint32_t)lane, (c + (uint32_t)lane) % (uint32_t)CH);
+#pragma unroll 1
+            for (uint64_t todo = __ballot(any); todo; todo &= todo - 1u) {
+                const uint32_t at = (uint32_t)__builtin_ctzll(todo);
+                const uint32_t slots = (uint32_t)__ballot(lane < CH && nonfinite(at, (uint32_t)lane % (uint32_t)CH));
+                float x = 0.0f;
+#pragma unroll
+                for (int j = 0; j < KS; ++j) {
+                    const half8_t kv = *(const half8_t*)(sb + at * HD + 8u * (((uint32_t)(2 * j + hf)) ^ ksw(at)));
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x = fmaf((float)qop[j][e], (float)kv[e], x);
+                }
+                x += __shfl_xor(x, 32);
+                const float p = fast_exp2(fmaf(x, a.scale_log2, -mref));
+                const bool sees = c0 + (int)at < lim;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int i = 0; i < 16; i += 4) {
+                        const uint32_t slot = (uint32_t)(4 * nb + i / 4) ^ vsw(at);
+                        if (!((slots >> slot) & 1u)) continue; // uniform
+                        const half4_t v = *(const half4_t*)(sb + OP + at * HD + 8u * slot + 4 * hf);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float f = (float)v[e];
+                            if (sees && !(fabsf(f) < INFINITY)) oacc[nb][i + e] = fmaf(p, f, oacc[nb][i + e]);
+                        }
+                    }
+            }
         }
     };
 
     constexpr short kWaitAll = (short)0x0070; // vmcnt(0), lgkmcnt(0): this wave's loads are in LDS, its LDS reads done
-    if (t0 < t1) {
+    auto pass = [&](auto split) {
+        m_run = -INFINITY;
+        l_run = 0.0f;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) oacc[nb] = (float16_t)0.0f;
+        if (t0 >= t1) return;
         issue(t0, 0);
         __builtin_amdgcn_s_waitcnt(kWaitAll);
         barrier();
         uint32_t buf = 0;
         for (uint32_t tt = t0; tt < t1; ++tt) {
             if (tt + 1u < t1) issue(tt + 1u, buf ^ 1u); // its readers (tile tt - 1) passed the previous barrier
-            process(tt, buf);
+            process(split, tt, buf);
             __builtin_amdgcn_s_waitcnt(kWaitAll);
             barrier();
             buf ^= 1u;
         }
-    }
-
-    const float l = l_run + __shfl_xor(l_run, 32);
-    // Rows with an inf or NaN among their sums (and finite weights), one at a time
-    // over the positions they see: in the tiles above, an inf or NaN value past a
-    // row's limit reaches the row as 0 * inf.
-    float chk = 0.0f;
+    };
+    pass(std::false_type{});
+    // An inf or NaN among the sums, under finite weights: it comes from the values, and
+    // may have reached rows that do not see it (0 * inf) or have a weight there that f16
+    // rounds to 0.  The work-group then takes its positions once more, split.  2048
+    // queries of 32/8 heads x 128 dims, us: finite values 66, one inf in each head 220
+    // (its rows one at a time without matrix instructions 10500), an inf at every
+    // position 1790; as groups of decodes 2920.
+    float l = l_run + __shfl_xor(l_run, 32), chk = 0.0f;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) chk = fmaf(oacc[nb][i], 0.0f, chk);
-    uint64_t redo = __ballot(chk != 0.0f && l * 0.0f == 0.0f && r < a.rows);
-    redo |= redo >> 32;
-    const bool done = (redo >> li) & 1u;
-    for (uint32_t todo = (uint32_t)redo; todo; todo &= todo - 1u)
-        prefill_row<HD>(a, g, s, wrow0 + (uint32_t)__builtin_ctz(todo), t0 * (uint32_t)kPrefillTokens, t1 * (uint32_t)kPrefillTokens);
-    if (done) return;
-    if (r >= a.rows) return;
+    uint32_t* flags = (uint32_t*)pre_lds; // every tile has been read
+    const bool redo = __any(chk != 0.0f && l * 0.0f == 0.0f && r < a.rows);
+    if (lane == 0) flags[wave] = redo ? 1u : 0u;
+    __syncthreads();
+    const uint32_t again = flags[0] | flags[1] | flags[2] | flags[3];
+    if (again) { // the same in every wave
+        __syncthreads();
+        pass(std::true_type{});
+        l = l_run + __shfl_xor(l_run, 32);
+    }
+    uint32_t ro = wrow0 + (uint32_t)li;
+    __asm__ volatile("" : "+v"(ro)); // its addresses are made here, not kept over the loops
+    if (ro >= a.rows) return;
     if (a.splits == 1u) {
         const float inv = l == 0.0f ? 0.0f : 1.0f / l;
-        uint16_t* po = a.out + ((uint64_t)qi * a.q_heads + head) * HD;
+        uint16_t* po = a.out + ((uint64_t)(ro / a.gqa) * a.q_heads + g * a.gqa + ro % a.gqa) * HD;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -316,7 +336,7 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
                 *(half4_t*)(po + 32 * nb + 2 * i + 4 * hf) = h;
             }
     } else {
-        const uint64_t at = ((uint64_t)g * a.splits + s) * a.rows + r;
+        const uint64_t at = ((uint64_t)g * a.splits + s) * a.rows + ro;
         if (hf == 0) {
             a.part_m[at] = m_run;
             a.part_l[at] = l;
