@@ -42,19 +42,33 @@ struct GemmTile {
     static_assert(NA >= 2 && (NB == NA || NB == NA + 1) && kLdsBytes <= 160 * 1024);
 };
 
-// Eight results C[m][n .. n+7] of one lane, masked to M x N; `vec` (N % 8 == 0, C
-// aligned to 16 bytes) reads and writes them 16 bytes at a time.
+// 16 bytes at an element's alignment: one access on gfx950, whatever row of an odd
+// length it lies in.
+typedef uint32_t uint4_a2_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef float float4_a4_t __attribute__((ext_vector_type(4), aligned(4)));
+
+// Eight results C[m][n .. n+7] of one lane, masked to M x N; all but the last of a row
+// whose N % 8 != 0 are read and written 16 bytes at a time.  4096 x N x 64, the stores
+// its bound, us with single values and this: N 8196 f16 80 -> 24, f32 106 -> 37,
+// residual 121 -> 51; N 8197 81 -> 41, 104 -> 48, 129 -> 72 (N 8192, 16 bytes at a
+// time both ways: 22, 28, 34).
 template <Epi EPI, bool F32>
 __device__ inline void store8(void* C, uint32_t M, uint32_t N, uint32_t m, uint32_t n, float4_t lo, float4_t hi,
-                              float scale, bool vec) {
-    if (!vec || F32) {
-        store4<EPI, F32>(C, M, N, m, n, lo, lo, scale, vec);
-        store4<EPI, F32>(C, M, N, m, n + 4u, hi, hi, scale, vec);
+                              float scale) {
+    if (n + 8 > N) {
+        store4<EPI, F32>(C, M, N, m, n, lo, lo, scale, false);
+        store4<EPI, F32>(C, M, N, m, n + 4u, hi, hi, scale, false);
         return;
     }
-    if (m >= M || n >= N) return;
-    uint4_t* at = (uint4_t*)((uint16_t*)C + (uint64_t)m * N + n);
-    uint4_t x = (uint4_t)0u, r;
+    if (m >= M) return;
+    if constexpr (F32) {
+        float* at = (float*)C + (uint64_t)m * N + n;
+        *(float4_a4_t*)at = lo * scale;
+        *(float4_a4_t*)(at + 4) = hi * scale;
+        return;
+    }
+    uint4_a2_t* at = (uint4_a2_t*)((uint16_t*)C + (uint64_t)m * N + n);
+    uint4_a2_t x = (uint4_a2_t)0u, r;
     if constexpr (EPI == Epi::Residual) x = *at;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
@@ -257,7 +271,7 @@ __global__ __launch_bounds__(T::kThreads) __attribute__((amdgpu_waves_per_eu(T::
 #pragma unroll
         for (int p = 0; p < FN / 2; ++p)
             store8<EPI, F32>(G.C, a.M, N, mrow + 16u * j, ncol + 32u * p + 8u * (uint32_t)lg, acc[2 * p][j],
-                             acc[2 * p + 1][j], a.scale, G.vec_out);
+                             acc[2 * p + 1][j], a.scale);
         if constexpr (FN % 2)
             store4<EPI, F32>(G.C, a.M, N, mrow + 16u * j, ncol + 16u * (FN - 1) + 4u * (uint32_t)lg, acc[FN - 1][j],
                              acc[FN - 1][j], a.scale, G.vec_out);

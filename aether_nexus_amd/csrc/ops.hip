@@ -101,10 +101,7 @@ double tile_us(const awo::GemmArgs& g, uint32_t n_cu) {
 template <typename T, bool F32, awo::Epi EPI>
 void launch_tile(const awo::GemmArgs& a, hipStream_t st) {
     awo::GemmArgs g = a;
-    for (uint32_t i = 0; i < g.groups; ++i) {
-        g.g[i].tiles = (uint32_t)cdiv64(g.g[i].N, T::TN);
-        g.g[i].vec_out = g.g[i].N % 8 == 0 && aligned(g.g[i].C, 16);
-    }
+    for (uint32_t i = 0; i < g.groups; ++i) g.g[i].tiles = (uint32_t)cdiv64(g.g[i].N, T::TN);
     hipLaunchKernelGGL((awo::gemm_tile_kernel<T, F32, EPI>), dim3((uint32_t)tile_count<T>(g)), dim3(T::kThreads),
                        T::kLdsBytes, st, g);
 }

@@ -371,6 +371,53 @@ def test_tiles_match_the_gathered_loads(ops, m, n, k):
     check_product(host(got[0][0])[rows], host(a)[rows], host(b), k, f"tiles {m}x{n}x{k}")
 
 
+@pytest.mark.parametrize("n", [8192, 8196, 8198, 8197])
+@pytest.mark.parametrize("off", [0, 1])
+def test_ragged_output_rows(ops, n, off):
+    """Output rows at every element alignment (N % 8 != 0, a buffer one element off): the
+    bits of the same columns of an aligned product, for the three stores, nothing
+    written past the end; and at most 2.5 times the aligned product's time where
+    the stores are the bound (16 bytes at odd addresses take 1.9 times an aligned
+    row's, one value at a time 3.5 and more)."""
+    import torch
+    m, k = 4096, 64
+    g = torch.Generator(device="cuda:0").manual_seed(n)
+    a, b = (torch.randn(s, generator=g, device="cuda:0").to(torch.float16) for s in ((m, k), (8200, k)))
+    x0 = torch.randn((m, 8200), generator=g, device="cuda:0").to(torch.float16)
+
+    def calls(w, at):
+        out = torch.full((m * w + at + 1,), float("nan"), dtype=torch.float16, device="cuda:0")
+        f32 = torch.full((m * w + at + 1,), float("nan"), dtype=torch.float32, device="cuda:0")
+        res = torch.full_like(out, float("nan"))
+        view = [t[at:at + m * w].view(m, w) for t in (out, f32, res)]
+        view[2].copy_(x0[:, :w])
+        ops.matmul(a, b, view[0], m, w, k)
+        ops.matmul_scaled(a, b, view[1], m, w, k, 0.25)
+        ops.matmul_add_residual(a, b, view[2], m, w, k, 0.5)
+        assert all(bool(torch.isnan(t[:at]).all()) and bool(torch.isnan(t[at + m * w:]).all()) for t in (out, f32, res))
+
+        def us(f):
+            best = float("inf")
+            for _ in range(6):
+                t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+                t[0].record()
+                for _ in range(10):
+                    f()
+                t[1].record()
+                torch.cuda.synchronize()
+                best = min(best, t[0].elapsed_time(t[1]) * 100)
+            return best
+        result = [t.clone() for t in view]
+        return result, [us(lambda: ops.matmul(a, b, view[0], m, w, k)),
+                        us(lambda: ops.matmul_scaled(a, b, view[1], m, w, k, 0.25))]
+    want, base = calls(8200, 0)
+    got, took = calls(n, off)
+    for t, w in zip(got, want):
+        assert torch.equal(t, w[:, :n])
+    print(f"{m} x {n} x {k}, {off} off: {took} us, aligned {base}", flush=True)
+    assert all(t < 2.5 * w for t, w in zip(took, base)), (took, base)
+
+
 def test_product_bits_do_not_depend_on_the_wave_count(ops):
     """A product takes 16 waves per weight tile when the tiles are few and 8 when
     they are many; the same rows give the same bits either way (the K partial
