@@ -15,8 +15,7 @@ constexpr int kStageK = 64; // k per LDS stage: a staged row is 128 bytes, eight
 
 // gfx9 buffer resource word 3 (32-bit data format) of the operand loads.
 constexpr uint32_t kRsrcWord3 = 0x00020000u;
-// The host keeps a tile's rows below 1 GiB, so an offset of 2 GiB plus any row's
-// lies past every tile: the load returns zeros.
+// An offset past every tile, whose rows the host keeps below 1 GiB: the load returns zeros.
 constexpr uint32_t kOutOfRange = 0x80000000u;
 constexpr uint64_t kTileBytesMax = 1ull << 30;
 

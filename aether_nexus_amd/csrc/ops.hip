@@ -163,7 +163,10 @@ int launch_products(aw_engine* e, const char* what, const uint16_t* a, const Pro
                     t.g[0] = g.g[i];
                     t.groups = 1;
                     const dim3 grid((uint32_t)cdiv64(t.g[0].N, awo::kTileN), (uint32_t)cdiv64(m, awo::kTileM));
-                    hipLaunchKernelGGL((awo::gemm_tiled_kernel<F32, EPI>), grid, dim3(256), 0, st, t);
+                    if (vec)
+                        hipLaunchKernelGGL((awo::gemm_tiled_kernel<true, F32, EPI>), grid, dim3(256), 0, st, t);
+                    else
+                        hipLaunchKernelGGL((awo::gemm_tiled_kernel<false, F32, EPI>), grid, dim3(256), 0, st, t);
                 }
             }
         }

@@ -423,14 +423,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(GemmArgs a) {
     }
 }
 
-// Products of more than 64 rows whose rows are not 16-byte aligned (or are over
-// 4 MiB): 128 x 128 output tiles, 4 waves of 64 x 64 (4 x 4 MFMA tiles each), k-steps
-// of 32 staged in LDS with the next step's loads in registers while the current step
-// is multiplied.  One weight matrix (group 0).  The steps are summed in the order of
-// gemm_tile_kernel, so both give the same bits.  Bound: the gathered loads.
+// Products of more than 64 rows whose rows are not 16-byte aligned (VEC false) or are
+// over 4 MiB (VEC, past the other kernel's buffer loads): 128 x 128 output tiles, 4 waves
+// of 64 x 64 (4 x 4 MFMA tiles each), k-steps of 32 staged in LDS with the next step's
+// loads in registers while the current step is multiplied.  One weight matrix (group 0).
+// The steps are summed in the order of gemm_tile_kernel, so both give the same bits.
+// Bound: the loads (65 x 128 x 2097216: 52 ms with 16-byte loads, 230 gathered).
 constexpr int kTileM = 128, kTileN = 128, kTileK = 32, kTilePitch = kTileK + 8; // halves per staged row
 
-template <bool F32, Epi EPI>
+template <bool VEC, bool F32, Epi EPI>
 __global__ __launch_bounds__(256) void gemm_tiled_kernel(GemmArgs a) {
     static_assert(EPI != Epi::SiluGate, "one weight matrix");
     __shared__ __attribute__((aligned(16))) _Float16 sB[2][kTileN * kTilePitch]; // weights
@@ -447,8 +448,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(GemmArgs a) {
         for (int j = 0; j < 2; ++j) {
             const int p = tid + 256 * j;
             const uint32_t r = (uint32_t)(p >> 2), k = k0 + 8u * (uint32_t)(p & 3);
-            pb[j] = piece<false>(B, min(n0 + r, N - 1u), a.K, k);
-            pa[j] = piece<false>(a.A, min(m0 + r, a.M - 1u), a.K, k);
+            pb[j] = piece<VEC>(B, min(n0 + r, N - 1u), a.K, k);
+            pa[j] = piece<VEC>(a.A, min(m0 + r, a.M - 1u), a.K, k);
         }
     };
     auto stage = [&](int buf, const half8_t (&pb)[2], const half8_t (&pa)[2]) {

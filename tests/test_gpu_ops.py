@@ -418,6 +418,31 @@ def test_ragged_output_rows(ops, n, off):
     assert all(t < 2.5 * w for t, w in zip(took, base)), (took, base)
 
 
+def test_rows_past_the_buffer_loads(ops):
+    """Rows just past 4 MiB, the longest that gemm_tile_kernel loads, keep 16-byte loads:
+    the bits of the gathered form, in at most half its time (42 ms of 170)."""
+    import torch
+    m, n, k = 65, 40, (1 << 21) + 64
+    g = torch.Generator(device="cuda:0").manual_seed(3)
+    a, b = (torch.randn((r, k), generator=g, device="cuda:0").to(torch.float16) for r in (m, n))
+    off = torch.empty(m * k + 1, dtype=torch.float16, device="cuda:0")[1:].view(m, k)
+    off.copy_(a)
+    got, ms = [], []
+    for x in (a, off):
+        out = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda:0")
+        ops.matmul_scaled(x, b, out, m, n, k, 0.5)
+        t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        t[0].record()
+        ops.matmul_scaled(x, b, out, m, n, k, 0.5)
+        t[1].record()
+        torch.cuda.synchronize()
+        got.append(out)
+        ms.append(t[0].elapsed_time(t[1]))
+    print(f"{m} x {n} x {k}: {ms[0]:.1f} ms, gathered {ms[1]:.1f}", flush=True)
+    assert bool(torch.isfinite(got[0]).all()) and torch.equal(got[0], got[1])
+    assert ms[0] < 0.5 * ms[1], ms
+
+
 def test_product_bits_do_not_depend_on_the_wave_count(ops):
     """A product takes 16 waves per weight tile when the tiles are few and 8 when
     they are many; the same rows give the same bits either way (the K partial
