@@ -969,18 +969,21 @@ int launch_prefill(aw_engine* e, const aw_decode_desc* d, uint32_t n, uint32_t k
     a.scale_log2 = d->scale * aw::kLog2e;
     const uint64_t items = (uint64_t)a.tiles * a.kv_heads;
     a.splits = prefill_splits(items, cdiv(kv_len, aw::kPrefillTokens), (uint64_t)a.kv_heads * a.rows, HD, e->n_cu);
-    const uint64_t part = (uint64_t)a.kv_heads * a.splits * a.rows;
-    const size_t stat = align_up(part * 4, kAlign), need = 2 * stat + part * HD * 4;
-    // A call being captured cannot grow the workspace: without parts it needs none.
-    if (a.splits > 1 && need > e->ws.cap && capturing(st)) a.splits = 1;
+    auto stat = [&] { return align_up((uint64_t)a.kv_heads * a.splits * a.rows * 4, kAlign); }; // bytes of part_m, part_l
+    auto need = [&] { return 2 * stat() + (uint64_t)a.kv_heads * a.splits * a.rows * HD * 4; };
+    // A call being captured cannot grow the workspace: as many parts as it holds, one
+    // needs none (17 queries of 32 heads over 4096 positions after an eager call over 700:
+    // a replay 100 us in one part, 29 so).
+    if (a.splits > 1 && need() > e->ws.cap && capturing(st))
+        while (a.splits > 1 && need() > e->ws.cap) a.splits /= 2;
     aw::MergeArgs m{};
     if (a.splits > 1) {
-        const int rc = ensure_keep(e->ws, need, e->retired_ws, e->last_error, st);
+        const int rc = ensure_keep(e->ws, need(), e->retired_ws, e->last_error, st);
         if (rc) return rc;
         char* ws = (char*)e->ws.ptr;
         a.part_m = (float*)ws;
-        a.part_l = (float*)(ws + stat);
-        a.part_o = (float*)(ws + 2 * stat);
+        a.part_l = (float*)(ws + stat());
+        a.part_o = (float*)(ws + 2 * stat());
     }
     {
         StageTimer t(e, AW_STAGE_HOT, st);

@@ -294,10 +294,17 @@ int aw_decode_device_noalloc(aw_engine* engine, const aw_decode_desc* desc, void
  * inference.rs:219,256-266).  Unlike the reference (threadgroup scores[4096],
  * ops.metal:564) kv_len is not limited to 4096: it may reach 4 Mi positions
  * (the hot-pool limit of aw_decode_device), and kv_len + 1 < num_queries is
- * rejected instead of wrapping.  Queries beyond 64 / (q_heads / kv_heads) per
- * call are processed in consecutive groups.  Like aw_decode_device, a call
- * being captured into a HIP graph cannot grow the engine's workspace or its
- * block table: make one eager call with that kv_len (or longer) first. */
+ * rejected instead of wrapping.  Up to 64 / (q_heads / kv_heads) queries run as
+ * one decode.  More run as tiles of 128 query rows of a kv head, whose positions
+ * are cut into parts (merged from the engine's workspace) where there are few
+ * rows; caches that are not 16-byte aligned take consecutive decodes instead.
+ * Like aw_decode_device, a call being captured into a HIP graph cannot grow the
+ * engine's workspace or its block table: make one eager call of that shape (or
+ * longer) first.  A captured call of more queries than one decode takes is not
+ * rejected without it, but records as many parts as the workspace holds then, down
+ * to one: the rounding of the eager call only where the workspace sufficed, and
+ * slower replays (17 queries of 32 heads over 4096 positions: 82 us in one part,
+ * 16 in 16). */
 int aw_multihead_attention_device(aw_engine* engine, const uint16_t* q, const uint16_t* k_cache,
                                   const uint16_t* v_cache, uint16_t* out, uint32_t kv_len,
                                   uint32_t head_dim, uint32_t q_heads, uint32_t kv_heads,

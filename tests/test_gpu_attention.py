@@ -599,3 +599,36 @@ def test_prompt_attention_infinite_value_cost(engine, stream, at):
         us.append(best)
     print(f"attention with an inf at {at}: {us[1]:.1f} us, without {us[0]:.1f}", flush=True)
     assert us[1] < 6 * us[0], us
+
+
+def test_prompt_attention_captured_with_a_small_workspace(stream):
+    """A captured call whose parts the workspace does not hold all takes those that it
+    holds: the oracle's result on every replay, faster than in one part."""
+    from aether_nexus_amd.weaver import WeaverEngine
+    nq, kv_len, hq, hkv, d = 17, 4096, 32, 8, 128
+    q, k, v = cache_case(21, nq, kv_len, hq, hkv, d, kv_len)
+    qt, kt, vt = (torch.from_numpy(x).cuda() for x in (q, k, v))
+    out, us = torch.empty_like(qt), []
+    ref = AO.multihead_attention_f64(q, k, v, kv_len, nq)
+    for warm in (0, 700):  # positions of an eager call before: none, fewer than the captured call's
+        with WeaverEngine() as eng:
+            if warm:
+                eng.multihead_attention(qt, kt, vt, out, warm, d, hq, hkv, nq, cache_tokens=kv_len)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                eng.multihead_attention(qt, kt, vt, out, kv_len, d, hq, hkv, nq, cache_tokens=kv_len)
+            best = float("inf")
+            for _ in range(4):
+                out.fill_(float("nan"))
+                torch.cuda.synchronize()
+                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                a.record()
+                graph.replay()
+                b.record()
+                torch.cuda.synchronize()
+                best = min(best, a.elapsed_time(b) * 1e3)
+                assert_close(out.double().cpu().numpy(), ref)
+            us.append(best)
+    print(f"captured 17 x 4096: {us[0]:.1f} us without a workspace, {us[1]:.1f} with one", flush=True)
+    assert us[1] < 0.7 * us[0], us
