@@ -47,7 +47,8 @@ def _checker(*names):
             return
         if tensor is None and t is not None and not isinstance(t, int):
             import torch
-            tensor, dtypes = torch.Tensor, tuple(getattr(torch, n) for n in names)
+            dtypes = tuple(getattr(torch, n) for n in names)
+            tensor = torch.Tensor  # last: another thread that sees it sees the dtypes
         _check_tensor(t, need, what, dtypes)
     return check
 

@@ -334,3 +334,30 @@ int main(void) {
 
 def lib_abi_version() -> int:
     return _lib.load().aw_abi_version()
+
+
+def test_tensor_checker_publishes_its_types_before_its_class():
+    """Another thread that calls a checker while its first tensor is looked at must not
+    refuse a good tensor: at every bytecode of that first call, once the class is
+    known to the checker the dtypes are too."""
+    import sys
+    import torch
+    from aether_nexus_amd import ops
+    check = ops._checker("float16", "int16")
+    cells = dict(zip(check.__code__.co_freevars, check.__closure__))
+    seen = []
+
+    def trace(frame, event, arg):
+        if frame.f_code is not check.__code__:
+            return None
+        frame.f_trace_opcodes = True
+        seen.append((cells["tensor"].cell_contents is not None, len(cells["dtypes"].cell_contents)))
+        return trace
+    old = sys.gettrace()
+    sys.settrace(trace)
+    try:
+        with pytest.raises(WeaverError):  # a tensor in host memory
+            check(torch.zeros(4, dtype=torch.float16), 4, "x")
+    finally:
+        sys.settrace(old)
+    assert (True, 2) in seen and (True, 0) not in seen
