@@ -241,3 +241,74 @@ def test_encode_resident_dictionary_edges(engine, stream, hkv, hd, a, dheads, nb
     assert (got == want).all(), f"{int((got != want).any(axis=-1).sum())} codes differ"
     scan, _ = run_device(engine, stream, hb, db, src, None, cold0.copy(), False, False, full_scan=True)
     assert (scan == want).all()
+
+
+@pytest.mark.parametrize("hkv,hd,a,nb", [(8, 128, 512, 1300), (16, 64, 1024, 520)])
+def test_encode_resident_dictionary_every_wave(engine, stream, hkv, hd, a, nb):
+    """More 64-token tiles than all waves of a head's work-groups (8 waves of 256 /
+    kv_heads work-groups on 256 CUs): every wave's list and a wave's second tile.
+    Stress tokens in blocks all over, all codes against the exact scan and
+    blocks of every wave's tiles against the oracle."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    wgs, tiles = cus // hkv, -(-nb * 16 // 64)
+    assert cus != 256 or tiles > 8 * wgs
+    rng = np.random.default_rng(nb)
+    hot = rng.standard_normal((nb, 16, hkv, hd)).astype(np.float16)
+    d = _unit(rng, (hkv, a, hd))
+    d[:, a - 3] = d[:, 11]
+    # One block in each wave's first tiles, and in second tiles: a wave's tiles start at wgs * wave.
+    blocks = sorted({4 * (wgs * w + p) + p % 4 for w in range(10) for p in (0, 7, wgs - 1)} & set(range(nb)) | {nb - 1})
+    for i, b in enumerate(blocks):
+        t = 1 + i % 14
+        hot[b, t] = 0
+        hot[b, t - 1, i % hkv, 3] = (np.inf, np.nan, -np.inf)[i % 3]
+        hot[b, t + 1] = np.float16(2.0 ** -20)
+        hot[b, (t + 7) % 16] = d[:, 11] * np.float16(3)  # two atoms tied for the best
+    hb, db = hot.view(np.uint16), d.view(np.uint16)
+    src, cold0 = np.arange(nb), np.zeros((nb, 16, hkv, 8), np.uint16)
+    rest = np.setdiff1d(src, blocks)
+    src[rest] = rng.permutation(rest)  # entry b decides its tile and wave: the stressed blocks stay put
+    print(f"encoder: resident dictionary, {tiles} tiles over {wgs} work-groups a head", flush=True)
+    got, _ = run_device(engine, stream, hb, db, src, None, cold0.copy(), False, False)
+    scan, _ = run_device(engine, stream, hb, db, src, None, cold0.copy(), False, False, full_scan=True)
+    assert (got == scan).all(), f"{int((got != scan).any(axis=-1).sum())} codes differ"
+    want = oracle.encode_blocks(hb, db, np.asarray(blocks), cold=cold0.copy())
+    assert (got[blocks] == want[blocks]).all()
+
+
+@pytest.mark.parametrize("hd,a", [(128, 528), (128, 576), (64, 1040), (64, 4096)])
+def test_encode_streamed_dictionary_stress(engine, stream, hd, a):
+    """The prefilter that streams a dictionary too large for LDS (a partial last chunk
+    of 64 atoms and none) on inputs built to stress it, one kind a head: inf and NaN
+    components, subnormal ones, atoms one f16 ulp apart, more tied atoms than a
+    candidate list holds.  Against the exact scan and the oracle, bit for bit."""
+    assert a * hd * 2 > 128 * 1024
+    rng = np.random.default_rng(a + hd)
+    hkv, nb = 4, 6
+    hot = rng.standard_normal((nb, 16, hkv, hd)).astype(np.float16)
+    d = _unit(rng, (hkv, a, hd))
+    d[0, 7, 3], d[0, 9, 0], d[0, a - 1, 5] = np.inf, np.nan, -np.inf
+    hot[1, 3, 0, 10], hot[2, 5, 0, 20], hot[3, 0, 0] = np.nan, np.inf, np.float16(-np.inf)
+    mask = rng.random(d[1].shape) < 0.05
+    d[1][mask] = (rng.choice([-1, 1], mask.sum()) * rng.integers(1, 1024, mask.sum()) * 2.0 ** -24).astype(np.float16)
+    mask = rng.random(hot[:, :, 1].shape) < 0.01
+    hot[:, :, 1][mask] = np.float16(2.0 ** -20)
+    x = hot[:, :, 2].reshape(-1, hd).astype(np.float32)
+    base = x[rng.choice(x.shape[0], 8, replace=False)]
+    base = (base / np.linalg.norm(base, axis=-1, keepdims=True)).astype(np.float16)
+    for k in range(8):
+        at = 8 * k if k < 4 else a - 8 * (k - 3)
+        d[2, at:at + 8] = base[k]
+        for j in range(1, 8):
+            d[2, at + j].view(np.uint16)[rng.integers(0, hd)] += np.uint16(1)
+    d[3, 40:80] = d[3, 3:4]  # 41 identical atoms
+    d[3, a - 30:] = d[3, 4:5]
+    hot[4, 2], hot[4, 3], hot[5, 9] = 0, np.float16(2.0 ** -24), d[:, 3] * np.float16(2)
+    hb, db, src = hot.view(np.uint16), d.view(np.uint16), rng.permutation(nb)
+    cold0 = np.zeros((nb, 16, hkv, 8), np.uint16)
+    print(f"encoder: streamed dictionary of {a} x {hd}", flush=True)
+    got, _ = run_device(engine, stream, hb, db, src, None, cold0.copy(), False, False)
+    scan, _ = run_device(engine, stream, hb, db, src, None, cold0.copy(), False, False, full_scan=True)
+    want = oracle.encode_blocks(hb, db, src, cold=cold0.copy())
+    assert (scan == want).all()
+    assert (got == want).all(), f"{int((got != want).any(axis=-1).sum())} codes differ"
