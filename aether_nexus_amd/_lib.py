@@ -42,6 +42,7 @@ SIGNATURES = {
     "aw_debug_project": (_c_int, [_vp, _vp, _vp, _vp]),
     "aw_multihead_attention_device": (_c_int, [_vp, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32, _u32, _u64, _vp]),
     "aw_engine_check_device_errors": (_c_int, [_vp, _vp]),
+    "aw_debug_product_tile": (_c_int, [_u32, _u32, _vp, _u32, _u32, _vp]),
     "aw_debug_gather_codes": (_c_int, [_vp, _vp, _sz, _vp, _u32, _u32, _vp, _vp, _vp, _vp]),
     "aw_engine_set_profiling": (_c_int, [_vp, _c_int]),
     "aw_engine_set_projection": (_c_int, [_vp, _c_int]),

@@ -98,6 +98,27 @@ double tile_us(const awo::GemmArgs& g, uint32_t n_cu) {
     return (double)rounds * ((double)cdiv64(g.K, awo::kStageK) * stage + 1.5 + area / 15e3);
 }
 
+// f(T{}) for the tile of the least estimate; false where no tile's grid fits.
+template <typename F>
+bool with_tile(const awo::GemmArgs& g, uint32_t n_cu, F f) {
+    double best = 0.0;
+    int pick = -1, i = 0;
+    each_tile([&](auto t) {
+        using T = decltype(t);
+        const double us = tile_us<T>(g, n_cu);
+        if (tile_count<T>(g) <= 0x7FFFFFFFull && (pick < 0 || us < best)) {
+            best = us;
+            pick = i;
+        }
+        ++i;
+    });
+    i = 0;
+    each_tile([&](auto t) {
+        if (i++ == pick) f(t);
+    });
+    return pick >= 0;
+}
+
 template <typename T, bool F32, awo::Epi EPI>
 void launch_tile(const awo::GemmArgs& a, hipStream_t st) {
     awo::GemmArgs g = a;
@@ -144,19 +165,8 @@ int launch_products(aw_engine* e, const char* what, const uint16_t* a, const Pro
         if constexpr (EPI != awo::Epi::SiluGate) {
             // 16-byte rows, a tile's rows below the buffer loads' limit.
             if (vec && (uint64_t)k * 512 <= awo::kTileBytesMax) {
-                const uint32_t n_cu = ei::compute_units(e);
-                double best = 0.0;
-                void (*launch)(const awo::GemmArgs&, hipStream_t) = nullptr;
-                each_tile([&](auto t) {
-                    using T = decltype(t);
-                    const double us = tile_us<T>(g, n_cu);
-                    if (tile_count<T>(g) <= 0x7FFFFFFFull && (!launch || us < best)) {
-                        best = us;
-                        launch = launch_tile<T, F32, EPI>;
-                    }
-                });
-                if (!launch) return ei::fail(e, AW_E_UNSUPPORTED, "%s: grid too large", what);
-                launch(g, st);
+                if (!with_tile(g, ei::compute_units(e), [&](auto t) { launch_tile<decltype(t), F32, EPI>(g, st); }))
+                    return ei::fail(e, AW_E_UNSUPPORTED, "%s: grid too large", what);
             } else {
                 for (uint32_t i = 0; i < g.groups; ++i) { // one launch per product, group 0 of its own arguments
                     awo::GemmArgs t = g;
@@ -398,6 +408,24 @@ int aw_ops_causal_attention(aw_engine* e, const uint16_t* q, const uint16_t* k, 
                             uint32_t kv_len, uint32_t head_dim, uint64_t cache_tokens, void* stream) {
     if (!e) return AW_E_INVALID_ARG;
     return aw_multihead_attention_device(e, q, k, v, output, kv_len, head_dim, 1, 1, 1, cache_tokens, stream);
+}
+
+int aw_debug_product_tile(uint32_t compute_units, uint32_t m, const uint32_t* n, uint32_t products, uint32_t k,
+                          uint32_t tile[3]) {
+    if (!n || !tile || products < 1 || products > 3 || m <= 64 || !compute_units) return AW_E_INVALID_ARG;
+    if (k % 8 || (uint64_t)k * 512 > awo::kTileBytesMax) return AW_E_UNSUPPORTED;
+    awo::GemmArgs g{};
+    g.M = m;
+    g.K = k;
+    for (uint32_t i = 0; i < products; ++i)
+        if (n[i]) g.g[g.groups++].N = n[i];
+    const bool ok = g.groups && with_tile(g, compute_units, [&](auto t) {
+        using T = decltype(t);
+        tile[0] = T::TM;
+        tile[1] = T::TN;
+        tile[2] = T::NB;
+    });
+    return ok ? AW_OK : AW_E_UNSUPPORTED;
 }
 
 } // extern "C"

@@ -130,6 +130,13 @@ int aw_ops_matmul_qkv(aw_engine* engine, const uint16_t* a, const uint16_t* b_q,
                       const uint16_t* b_v, uint16_t* q, uint16_t* k_out, uint16_t* v_out, uint32_t m, uint32_t n_q,
                       uint32_t n_kv, uint32_t k, void* hip_stream);
 
+/* The tile that a call's product (matmul_qkv: 3, of n[0 .. products) weight rows)
+ * of m > 64 rows with 16-byte aligned rows takes on a GPU of `compute_units`, for
+ * testing: {activation rows, weight rows, LDS buffers of 64 k}.  Host only.
+ * AW_E_UNSUPPORTED where such a product takes none (k % 8 != 0, k > 2 Mi). */
+int aw_debug_product_tile(uint32_t compute_units, uint32_t m, const uint32_t* n, uint32_t products, uint32_t k,
+                          uint32_t tile[3]);
+
 #ifdef __cplusplus
 }
 #endif

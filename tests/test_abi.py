@@ -361,3 +361,15 @@ def test_tensor_checker_publishes_its_types_before_its_class():
     finally:
         sys.settrace(old)
     assert (True, 2) in seen and (True, 0) not in seen
+
+
+def test_debug_product_tile():
+    """The tile of a product on 256 CUs, without a GPU; what it refuses."""
+    lib, tile = _lib.load(), (ctypes.c_uint32 * 3)()
+
+    def ask(m, k, *n, products=None):
+        return lib.aw_debug_product_tile(256, m, (ctypes.c_uint32 * 3)(*n), len(n) if products is None else products, k, tile)
+    assert ask(2048, 4096, 14336) == 0 and tuple(tile) == (256, 256, 3)
+    assert ask(117, 2048, 2048, 512, 512) == 0 and tuple(tile) == (64, 32, 6)
+    assert ask(64, 4096, 4096) == ask(65, 64, 64, products=4) == ask(65, 64, 64, products=0) == AW_E_INVALID_ARG
+    assert ask(65, 12, 64) == ask(65, (1 << 21) + 8, 64) == ask(65, 64, 0) == AW_E_UNSUPPORTED

@@ -183,6 +183,39 @@ def test_rope(ops, tokens, hq, hkv, hd, start):
         assert np.array_equal(bits(host(tk)), bits(k))  # no k heads: untouched
 
 
+# (tokens, q heads, kv heads, dims, heads a thread takes on 256 CUs): a group across the last q
+# heads and the first k heads, a last group of fewer heads, no k heads, a few odd dims, all heads of a
+# token in one thread.
+ROPE_GROUPS = [(512, 32, 8, 128, 8), (700, 14, 2, 64, 2), (740, 12, 2, 128, 5), (1200, 12, 2, 128, 8), (300, 32, 0, 128, 4),
+               (30000, 2, 2, 6, 2), (4096, 2, 1, 128, 6)]
+
+
+@pytest.mark.parametrize("tokens,hq,hkv,hd,per", ROPE_GROUPS, ids=["-".join(map(str, c)) for c in ROPE_GROUPS])
+def test_rope_several_heads_a_thread(ops, tokens, hq, hkv, hd, per):
+    """Enough tokens for a thread to turn several heads: the bits of calls of so few
+    tokens that each thread has one, and the oracle's values on some tokens."""
+    import torch
+    start, theta, heads, pairs = 4097, 500000.0, hq + hkv, hd // 2
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    if cus == 256:
+        assert per == min(8, tokens * pairs * heads // (512 * cus))
+    g = torch.Generator(device="cuda:0").manual_seed(tokens)
+    q, k = (torch.randn((tokens, max(h, 1), hd), generator=g, device="cuda:0").to(torch.float16) for h in (hq, hkv))
+    q0, k0 = q.clone(), k.clone()
+    wq, wk = q.clone(), k.clone()
+    ops.rope(q, k if hkv else None, tokens, hq, hkv, hd, start, theta)
+    few = 1024 * cus // (pairs * heads) - 1
+    for t in range(0, tokens, few):
+        n = min(few, tokens - t)
+        ops.rope(wq[t:t + n], wk[t:t + n] if hkv else None, n, hq, hkv, hd, start + t, theta)
+    assert torch.equal(q.view(torch.int16), wq.view(torch.int16)) and torch.equal(k.view(torch.int16), wk.view(torch.int16))
+    assert hkv or torch.equal(k, k0)
+    for t in (0, tokens // 2, tokens - 1):
+        for x, x0 in ((q, q0), (k, k0))[:2 if hkv else 1]:
+            within_one_ulp(host(x[t:t + 1]).reshape(1, -1, hd), O.rope_f32(host(x0[t:t + 1]).reshape(1, -1, hd), start + t, theta),
+                           f"rope token {t}")
+
+
 # M <= 16, 32, 64 take the skinny kernel with 1, 2, 4 row tiles (16 waves up to 4 weight tiles per CU, 8
 # beyond: N = 20000 and 49155), larger M the tiled one; K % 8 != 0 the element-wise loads.
 # 256 x 128 tiles where they fill the CUs: 1000 x 8200 x 520 (ragged M, N and a partial
@@ -336,7 +369,7 @@ def test_wide_and_tiled_products_same_bits(ops, k):
 
 # A shape that takes each tile of gemm_tile_kernel (256 x 256, 256 x 160, 256 x 128, 128 x 128,
 # 128 x 64, 64 x 96, 64 x 64, 64 x 32), ragged in M and N (8-wide stores and not), with one stage of
-# K, a partial one, fewer than the tile's LDS buffers and more.
+# K, a partial one, and for most tiles no more stages than LDS buffers (LONG_TILES has more for each).
 TILE_SHAPES = [(2000, 8008, 200), (1000, 8200, 520), (500, 14001, 72), (700, 5000, 72), (200, 8190, 136),
                (300, 4868, 128), (300, 2056, 1032), (65, 96, 264), (129, 1, 8), (66, 33, 64), (8400, 40, 24)]
 
@@ -369,6 +402,26 @@ def test_tiles_match_the_gathered_loads(ops, m, n, k):
         assert bool(torch.isfinite(t).all()) and torch.equal(t, w), i
     rows = torch.unique(torch.cat([torch.arange(min(m, 16)), torch.tensor([m // 2, m - 1])]))
     check_product(host(got[0][0])[rows], host(a)[rows], host(b), k, f"tiles {m}x{n}x{k}")
+
+
+# (m, n, k, tile): each tile with more than twice as many stages of K as LDS buffers, the last one
+# partial, ragged in M and N.
+LONG_TILES = [(1029, 8167, 456, (256, 256)), (772, 8477, 456, (256, 160)), (388, 8438, 456, (256, 128)),
+              (131, 8201, 456, (128, 128)), (145, 8170, 472, (128, 64)), (65, 8389, 536, (64, 96)),
+              (71, 4321, 520, (64, 64)), (84, 39, 1016, (64, 32))]
+
+
+@pytest.mark.parametrize("m,n,k,tile", LONG_TILES, ids=[f"{c[3][0]}x{c[3][1]}" for c in LONG_TILES])
+def test_each_tile_past_its_buffers(ops, m, n, k, tile):
+    """The steady loop of every tile, its LDS buffers used again, in all three stores and
+    q/k/v; that the tile is the one meant."""
+    import ctypes
+    import torch
+    got = (ctypes.c_uint32 * 3)()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert ops._lib.aw_debug_product_tile(cus, m, (ctypes.c_uint32 * 1)(n), 1, k, got) == 0
+    assert tuple(got[:2]) == tile and -(-k // 64) > 2 * got[2], tuple(got)
+    test_tiles_match_the_gathered_loads(ops, m, n, k)
 
 
 @pytest.mark.parametrize("n", [8192, 8196, 8198, 8197])
