@@ -549,7 +549,7 @@ def encoder_bench(engine, seed, reps, cpu_blocks):
     tf = flops / (ms * 1e-3) / 1e12
     scan_tf = flops / (scan_ms * 1e-3) / 1e12
     return {"workload": f"{nb} blocks x 16 tokens x {hkv} kv heads, head_dim {hd}, {a} atoms per kv head, "
-                        "entropy proxy included (on a side stream beside the encoder)",
+                        "entropy proxy included (on a side stream; the encoder's work-groups hold every CU, so it runs after them)",
             "ms_per_call": round(ms, 4), "blocks_per_s": round(nb / (ms * 1e-3), 1),
             "token_heads_per_s": round(tok_heads / (ms * 1e-3), 1),
             "achieved_tflops": round(tf, 2),
